@@ -15,6 +15,8 @@
 #include "capi_common.hpp"
 #include "device_common.hpp"
 #include "plan.hpp"
+#include "row_plan.hpp"
+#include "row_solve.hpp"
 
 namespace g2g {
 
@@ -160,6 +162,58 @@ struct g2g_plan_s {
     } dx;
     bool ext() const { return grid && nr.xt.on(); }
     int prog_f_stride = 0, prog_b_stride = 0;
+    // row solver: the host tables' sizes (RowPlan without its large arrays) and
+    // their device copy, one allocation made with the first batch
+    struct {
+        bool tried = false;
+        RowPlan r;
+        unsigned char* buf = nullptr;
+        const int *bus_of = nullptr, *lev_ptr = nullptr, *rec_ptr = nullptr, *rec = nullptr, *rec2 = nullptr,
+                  *term = nullptr, *back = nullptr, *back_col = nullptr, *fill = nullptr, *slice_ptr = nullptr,
+                  *slice_bus = nullptr, *ent = nullptr;
+        const double *ent_y = nullptr, *diag_y = nullptr;
+    } rw;
+    void upload_rows()
+    {
+        if (rw.tried || !grid || nr.xt.on()) return;
+        rw.tried = true;
+        RowPlan r = build_row_plan(nr);
+        if (!r.ok) return;
+        std::vector<unsigned char> h;
+        std::vector<std::pair<const void**, size_t>> parts;
+        auto add = [&](auto& ptr, const auto& v) {  // (an empty table still has an address)
+            parts.push_back({reinterpret_cast<const void**>(&ptr), h.size()});
+            const size_t bytes = v.size() * sizeof(v[0]);
+            h.resize((h.size() + bytes + 63) / 64 * 64 + 64);
+            if (bytes) std::memcpy(h.data() + parts.back().second, v.data(), bytes);
+        };
+        add(rw.bus_of, r.bus_of);
+        add(rw.lev_ptr, r.lev_ptr);
+        add(rw.rec_ptr, r.rec_ptr);
+        add(rw.rec, r.rec);
+        add(rw.rec2, r.rec2);
+        add(rw.term, r.term);
+        add(rw.back, r.back);
+        add(rw.back_col, r.back_col);
+        add(rw.fill, r.fill);
+        add(rw.slice_ptr, r.slice_ptr);
+        add(rw.slice_bus, r.slice_bus);
+        add(rw.ent, r.ent);
+        add(rw.ent_y, r.ent_y);
+        add(rw.diag_y, r.diag_y);
+        rw.buf = dupload(h);
+        for (const auto& q : parts) *q.first = rw.buf + q.second;
+        rw.r.n_fill = r.n_fill;
+        rw.r.n = r.n;
+        rw.r.nb = r.nb;
+        rw.r.n_blk = r.n_blk;
+        rw.r.n_lev = r.n_lev;
+        rw.r.n_slice = r.n_slice;
+        rw.r.solo_f = r.solo_f;
+        rw.r.solo_b = r.solo_b;
+        rw.r.lev_blk = r.lev_blk;
+        rw.r.ok = true;
+    }
     bool uploaded = false;
     const SymbolicLU& lu() const { return grid ? nr.lu : raw; }
     ~g2g_plan_s()
@@ -169,6 +223,7 @@ struct g2g_plan_s {
         dfree(d_colmap); dfree(d_entry_row);
         dfree(d_k1_ent_t);
         dx.free_all();
+        dfree(rw.buf);
         dfree(d_prog_fs); dfree(d_prog_bs); dfree(d_split_seg); dfree(d_split_bseg); dfree(d_k1_bus_s);
         dfree(d_k1_ent_s);
     }
@@ -321,7 +376,7 @@ struct g2g_batch_s {
     int* n_active = nullptr;  // rows and tiles still iterating (2 ints)
     int* clamped = nullptr;
     int* error = nullptr;     // stream kernels' give-up flag
-    int* h_active = nullptr;  // pinned: rows and tiles still iterating, rows restarted
+    int* h_active = nullptr;  // pinned: rows and tiles still iterating, rows restarted; [4..8]: row_cnt
     // warm solves: the caller's start voltages (the fallback start)
     double2* V0 = nullptr;
     bool v0_row = false;  // V0 holds one row [n] (every row's fallback start is the same)
@@ -404,6 +459,12 @@ struct g2g_batch_s {
     // so a refill or a take allocates and frees nothing once warm)
     void* stage[kStageBufs] = {};
     size_t stage_cap[kStageBufs] = {};
+    // row solver: per-workgroup scratch (grown on use), the active rows' list,
+    // and its counters {Newton updates (64 bits), largest iteration, list length, rows left}
+    unsigned char* row_scratch = nullptr;
+    size_t row_scratch_cap = 0;
+    int* row_list = nullptr;
+    int* row_cnt = nullptr;
     std::vector<hipEvent_t> ev;
     ~g2g_batch_s()
     {
@@ -420,6 +481,7 @@ struct g2g_batch_s {
         dfree(mask); dfree(maskk); dfree(xs); dfree(xsk); dfree(sx); dfree(pend);
         dfree(budget); dfree(warm); dfree(requeued); dfree(V0k); dfree(it0k); dfree(budgetk); dfree(warmk);
         for (void*& q : stage) dfree(q);
+        dfree(row_scratch); dfree(row_list); dfree(row_cnt);
         if (h_active) (void)hipHostFree(h_active);
         for (auto e : ev) (void)hipEventDestroy(e);
     }
@@ -1349,6 +1411,210 @@ void zero_a_tiles(g2g_batch_s* b, int T)
     b->split_T = std::max(b->split_T, T);
 }
 
+// ---- the row solver (row_solve.hip) ---------------------------------------
+
+// G2G_ROWS=0 / 1: never / whenever the row solver can run.  An override of
+// the tile kernels' shape (the other variables) keeps a solve on them.
+int rows_env()
+{
+    if (const char* e = std::getenv("G2G_ROWS")) return std::atoi(e) ? 1 : 0;
+    for (const char* v : {"G2G_SPLIT", "G2G_COMPACT", "G2G_MIS_SPLITS", "G2G_WALKERS", "G2G_BWALKERS",
+                          "G2G_HALF_RINGS", "G2G_IR_REFACTOR"})
+        if (std::getenv(v)) return 0;
+    return -1;
+}
+
+struct RowShape {
+    bool ok = false, blk_lds = false, v_lds = false;
+    int threads = 0, per_cu = 1, lds0 = 0, lev_lds = 0;
+    size_t lds = 0, scratch = 0;
+};
+
+// The workgroup's shape for R rows: V and every block in LDS where they fit;
+// else as many of the highest levels' blocks as fit, the rest (and V) in
+// scratch, with two workgroups a CU once there is more than a row a CU.
+template <typename Real>
+RowShape row_shape(const g2g_batch_s* b, int R)
+{
+    RowShape s;
+    const RowPlan& r = b->plan->rw.r;
+    if (!r.ok) return s;
+    const size_t limit = lds_limit();
+    const bool ed = b->per_row_y != 0;
+    const size_t all = static_cast<size_t>(r.n_blk) * 4 * sizeof(Real);
+    const size_t with_v = row_lds_bytes<Real>(r.n, r.nb, true, ed), no_v = row_lds_bytes<Real>(r.n, r.nb, false, ed);
+    // threads: enough that the widest levels are a few records a thread (997
+    // buses FP64, 12,288 rows: 512 threads 10.4 ms, 256 11.7; 2,000 mixed, 8,192
+    // rows: 1,024 6.8 ms, 512 7.1), few where several workgroups share a CU
+    // (118 buses, 16,384 rows: 128 1.09 ms, 256 1.72)
+    s.threads = r.nb <= 64 ? 64 : r.nb <= 300 ? 128 : r.nb <= 600 ? 256 : r.nb <= 1500 ? 512 : 1024;
+    if (with_v + all <= limit) {
+        s.blk_lds = s.v_lds = true;
+        s.lds = with_v + all;
+    } else if (no_v + all <= limit) {
+        s.blk_lds = true;
+        s.lds = no_v + all;
+    } else {
+        const size_t room = R > b->n_cu && 2 * no_v <= limit && 2 * s.threads <= 2048 ? limit / 2 : limit;
+        s.v_lds = 2 * with_v <= room;
+        const size_t base = s.v_lds ? with_v : no_v;
+        if (base > room) return s;
+        const size_t fit = (room - base) / (4 * sizeof(Real));
+        s.lds0 = r.n_blk - static_cast<int>(fit);
+        s.lds = base + fit * 4 * sizeof(Real);
+        while (r.lev_blk[s.lev_lds] < s.lds0) ++s.lev_lds;
+    }
+    s.per_cu = std::max(1, std::min<int>(static_cast<int>(limit / s.lds), 2048 / s.threads));
+    s.scratch = row_scratch_bytes<Real>(r.n, r.nb, s.lds0, s.v_lds, b->ir_steps > 0);
+    s.ok = true;
+    return s;
+}
+
+// Whether the solver's options allow the row solver at all.
+bool rows_possible(const g2g_batch_s* b)
+{
+    return b->plan->rw.r.ok && !b->mask && !b->xs && b->max_dva <= 0.0 && (b->ir_steps == 0 || b->ir_fp64) &&
+           !(b->per_row_y && b->ed_cap > kRowMaxEdits);
+}
+
+template <typename Real>
+bool use_rows(const g2g_batch_s* b, int active_rows)
+{
+    if (active_rows <= 0 || !rows_possible(b)) return false;
+    const RowShape s = row_shape<Real>(b, active_rows);
+    if (!s.ok) return false;
+    const int env = rows_env();
+    if (env >= 0) return env == 1;
+    // Where the two cross over, measured per solve (tile kernels / row solver):
+    // 118 buses FP64 16,384 rows 1.73 / 1.09 ms (the row solver at any count: several workgroups a CU);
+    // 997 FP64 12,288 rows 12.1 / 10.4 ms; 2,000 mixed 12,288 rows 10.6 / 10.2, 8,192 10.4 / 6.8 (one a CU);
+    // 2,000 FP64 (200 KB of scratch a workgroup, in the L2 and last-level cache) 4,096 rows 8.9 / 6.4, 8,192 15.1 / 12.9;
+    // 6,500 mixed (420 KB) 1,024 rows 7.0 / 6.2, 2,048 11.3 / 12.2; 6,500 FP64 (900 KB) 768 rows 10.1 / 7.4, 1,024 10.7 / 10.5
+    if (s.blk_lds && s.per_cu >= 4) return true;
+    return active_rows <= b->n_cu * (s.blk_lds ? 48 : s.scratch <= (256u << 10) ? 24 : s.scratch <= (512u << 10) ? 4 : 3);
+}
+
+template <typename Real, bool BL, bool VL>
+void launch_row_kernel(const RowShape& s, const RowArgs<Real>& a, int grid, hipStream_t st)
+{
+    HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_row_solve<Real, BL, VL>),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(s.lds)));
+    k_row_solve<Real, BL, VL><<<grid, s.threads, s.lds, st>>>(a);
+    HIPCHK(hipGetLastError());
+}
+
+constexpr int kRowCnt = 5;
+
+// Runs the R active rows from iteration `it` to their end; last_iter: the
+// largest iteration count.  decided: the statuses of iteration `it` already
+// stand (the mismatch there has run).  Returns the rows left as they came
+// (still active, nothing of theirs written).
+template <typename Real>
+int solve_rows(g2g_batch_s* b, int R, int it, bool decided, int max_iter, double tol, int freeze, double growth,
+               SolveTimer& tm, long long& rows_factored, int& last_iter)
+{
+    const g2g_plan_s* P = b->plan;
+    const RowPlan& r = P->rw.r;
+    const RowShape s = row_shape<Real>(b, R);
+    hipStream_t st = b->stream;
+    const int e0 = tm.mark();
+    const int grid = std::min(R, b->n_cu * s.per_cu);
+    const size_t need = s.scratch * static_cast<size_t>(grid);
+    if (need > b->row_scratch_cap) {
+        dfree(b->row_scratch);
+        b->row_scratch = nullptr;
+        b->row_scratch_cap = 0;
+        b->row_scratch = dalloc<unsigned char>(need);
+        b->row_scratch_cap = need;
+    }
+    if (!b->row_cnt) b->row_cnt = dalloc<int>(kRowCnt);
+    k_fill_int<<<1, 64, 0, st>>>(b->row_cnt, 0, kRowCnt);
+    const bool listed = R < b->active_rows;
+    if (listed) {
+        if (!b->row_list) b->row_list = dalloc<int>(static_cast<size_t>(b->rows_pad));
+        k_collect_rows<<<blocks_for(b->active_rows, 256), 256, 0, st>>>(b->status, b->active_rows, b->row_list,
+                                                                        b->row_cnt + 3);
+        HIPCHK(hipGetLastError());
+    }
+    RowArgs<Real> a{};
+    a.n = r.n;
+    a.nb = r.nb;
+    a.n_blk = r.n_blk;
+    a.n_lev = r.n_lev;
+    a.n_slice = r.n_slice;
+    a.n_fill = r.n_fill;
+    a.solo_f = r.solo_f;
+    a.solo_b = r.solo_b;
+    a.blk_lds0 = s.lds0;
+    a.lev_lds = s.lev_lds;
+    a.bus_of = P->rw.bus_of;
+    a.lev_ptr = P->rw.lev_ptr;
+    a.rec_ptr = P->rw.rec_ptr;
+    a.rec = reinterpret_cast<const int4*>(P->rw.rec);
+    a.rec2 = reinterpret_cast<const int2*>(P->rw.rec2);
+    a.term = reinterpret_cast<const int2*>(P->rw.term);
+    a.back = reinterpret_cast<const int4*>(P->rw.back);
+    a.back_col = P->rw.back_col;
+    a.fill = P->rw.fill;
+    a.slice_ptr = P->rw.slice_ptr;
+    a.slice_bus = reinterpret_cast<const int4*>(P->rw.slice_bus);
+    a.ent = reinterpret_cast<const int4*>(P->rw.ent);
+    a.ent_y = reinterpret_cast<const double2*>(P->rw.ent_y);
+    a.diag_y = reinterpret_cast<const double2*>(P->rw.diag_y);
+    a.V = b->V;
+    a.S = b->S;
+    if (b->per_row_y) a.ed = row_edits(b);
+    a.entry_row = P->d_entry_row;
+    a.status = b->status;
+    a.iters = b->iters;
+    a.res = b->res;
+    a.jmax = b->jmax;
+    a.rows = b->active_rows;
+    a.list = listed ? b->row_list : nullptr;
+    a.list_n = b->row_cnt + 3;
+    a.iter0 = it;
+    a.skip_first = decided ? 1 : 0;
+    a.max_iter = max_iter;
+    a.tol = tol;
+    a.freeze = freeze;
+    a.growth = growth;
+    a.contraction = b->contraction;
+    a.pivot_eps = b->precision == G2G_MIXED ? 1e-5 : 1e-12;
+    a.ir_steps = b->ir_steps;
+    if (b->restart_on) {
+        a.it0 = b->it0;
+        a.budget = b->budget;
+        a.warm = b->warm;
+        a.V0 = b->V0;
+        a.v0_row = b->v0_row ? 1 : 0;
+        a.restart_max_iter = b->restart_max_iter;
+        a.requeued = b->requeued;
+    }
+    a.scratch = b->row_scratch;
+    a.scratch_stride = s.scratch;
+    a.updates = reinterpret_cast<unsigned long long*>(b->row_cnt);
+    a.last_iter = b->row_cnt + 2;
+    a.left = b->row_cnt + 4;
+    if (s.blk_lds && s.v_lds) launch_row_kernel<Real, true, true>(s, a, grid, st);
+    else if (s.blk_lds) launch_row_kernel<Real, true, false>(s, a, grid, st);
+    else if (s.v_lds) launch_row_kernel<Real, false, true>(s, a, grid, st);
+    else launch_row_kernel<Real, false, false>(s, a, grid, st);
+    tm.ph[1].push_back({e0, tm.mark()});
+    tm.factor_main.push_back(0);
+    HIPCHK(hipMemcpyAsync(b->h_active + 4, b->row_cnt, kRowCnt * sizeof(int), hipMemcpyDeviceToHost, st));
+    HIPCHK(hipStreamSynchronize(st));
+    unsigned long long upd = 0;
+    std::memcpy(&upd, b->h_active + 4, sizeof(upd));
+    rows_factored += static_cast<long long>(upd);
+    last_iter = std::max(last_iter, b->h_active[6]);
+    const int left = b->h_active[8];
+    if (left > 0) {
+        k_count_tiles<<<b->T, kLanes, 0, st>>>(b->status, b->rows_pad, b->tile_active);
+        HIPCHK(hipGetLastError());
+    }
+    return left;
+}
+
 template <typename Real>
 int nr_loop_body(g2g_batch_s* b, int max_iter, double tol, int freeze, double growth, SolveTimer& tm,
                  long long& rows_factored, bool& compacted)
@@ -1361,6 +1627,14 @@ int nr_loop_body(g2g_batch_s* b, int max_iter, double tol, int freeze, double gr
     }
     int it = 0;
     int restarts = 0;
+    int last_row_iter = 0;      // of the rows the row solver finished
+    bool rows_tried = false;
+    if (use_rows<Real>(b, b->active_rows)) {
+        rows_tried = true;
+        if (solve_rows<Real>(b, b->active_rows, 0, false, max_iter, tol, freeze, growth, tm, rows_factored,
+                             last_row_iter) == 0)
+            return last_row_iter;
+    }
     for (;; ++it) {
         k_fill_int<<<1, 64, 0, b->stream>>>(b->n_active, 0, 2);
         int e0 = tm.mark();
@@ -1394,6 +1668,16 @@ int nr_loop_body(g2g_batch_s* b, int max_iter, double tol, int freeze, double gr
             tm.ph[0].push_back({e0, tm.mark()});
         }
         if (*b->h_active == 0) break;
+        // few rows left: the row solver takes them to their end, from the
+        // batch's own layout
+        if (!rows_tried && use_rows<Real>(b, b->h_active[0])) {
+            rows_tried = true;
+            const int left = solve_rows<Real>(b, b->h_active[0], it, true, max_iter, tol, freeze, growth, tm,
+                                              rows_factored, last_row_iter);
+            if (left == 0) return std::max(it, last_row_iter);
+            b->h_active[0] = left;
+            b->h_active[1] = std::min(left, live_tiles(b));
+        }
         if (worth_compacting(b, b->h_active[0], b->h_active[1])) {
             // (again: the rows go back to their batch places first)
             if (compacted) uncompact_rows(b);
@@ -1443,7 +1727,7 @@ int nr_loop_body(g2g_batch_s* b, int max_iter, double tol, int freeze, double gr
         launch_ext_update<Real>(b);
         tm.ph[2].push_back({e0, tm.mark()});
     }
-    return it;
+    return std::max(it, last_row_iter);
 }
 
 // Newton iterations on the batch's active rows until none is left or the
@@ -1627,7 +1911,7 @@ void solve_impl(g2g_batch_s* b, int max_iter, double tol, int sched, g2g_solve_s
     b->streaming = false;
     reset_rows(b);
     launch_ext_init<Real>(b);
-    SolveTimer tm(b, 3 * (max_iter + 1) + 2);
+    SolveTimer tm(b, 3 * (max_iter + 1) + 4);
     const int e_begin = tm.mark();
     long long rows_factored = 0;
     const int it = nr_loop<Real>(b, max_iter, tol, freeze, 0.0, tm, rows_factored);
@@ -2206,6 +2490,7 @@ int g2g_batch_create(g2g_plan_t P, int32_t rows, int32_t precision, int32_t per_
         if (precision != G2G_FP64 && precision != G2G_MIXED) throw std::invalid_argument("unknown precision");
         P = plan_fitting(P, precision == G2G_FP64);
         P->upload();
+        P->upload_rows();
         auto b = std::make_unique<g2g_batch_s>();
         b->plan = P;
         b->rows = b->active_rows = rows;
@@ -2270,7 +2555,7 @@ int g2g_batch_create(g2g_plan_t P, int32_t rows, int32_t precision, int32_t per_
         b->n_active = dalloc<int>(4);  // rows, tiles; a partial pass's spare pair
         b->error = dalloc<int>(1);
         HIPCHK(hipMemsetAsync(b->error, 0, sizeof(int), b->stream));
-        HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&b->h_active), 4 * sizeof(int), hipHostMallocDefault));
+        HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&b->h_active), 16 * sizeof(int), hipHostMallocDefault));
         k_fill_int<<<blocks_for(rp, 256), 256, 0, b->stream>>>(b->status, kNotSimulated, rp);
         k_fill_int<<<blocks_for(rp, 256), 256, 0, b->stream>>>(b->iters, 0, rp);
         HIPCHK(hipGetLastError());

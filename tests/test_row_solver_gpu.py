@@ -1,0 +1,170 @@
+"""The row solver (one workgroup per power flow) against the tile kernels
+(G2G_ROWS=0) and the CPU oracle, at the edges of its shapes: the smallest
+grids (one bus with unknowns, one elimination level), fixed buses, every block
+and V in LDS, the blocks alone, part of the blocks; one row, partial tiles,
+more rows than workgroups; edited Ybus rows, learned starts with restarts,
+refinement, both schedules; and rows that do not converge, which it leaves to
+the tile kernels."""
+import sys
+
+import numpy as np
+import pytest
+
+from gpusim2grid_amd import _capi
+from gpusim2grid_amd import synthetic as syn
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+
+def _grid(n):
+    if n in (2, 3):
+        return syn.make_grid(n, n - 1, n_pv=n - 2, accept=False)
+    named = {14: syn.grid_c0, 118: syn.grid_118, 2000: syn.grid_c1, 6500: syn.grid_c2}
+    return named[n]() if n in named else syn.make_grid(n, (3 * n) // 2, pv_frac=0.15)
+
+
+def _solve(g, S, prec, monkeypatch, rows_on, pv=None, pq=None, edits=None, ir=0, sched=_capi.CONTINUOUS, max_iter=10):
+    print(f"row solver n={g.n_bus} rows={S.shape[0]} prec={prec} rows_on={rows_on} ir={ir}", flush=True)
+    sys.stdout.flush()
+    monkeypatch.setenv("G2G_ROWS", str(rows_on))
+    P = _capi.Plan.from_grid(g.Ybus, g.pv if pv is None else pv, g.pq if pq is None else pq, g.slack)
+    B = _capi.Batch(P, S.shape[0], precision=prec, per_row_ybus=edits is not None)
+    if ir:
+        B.set_step_control(ir_steps=ir)
+        B.set_refinement_residual(True)
+    B.set_sbus(S)
+    B.set_v(g.flat_start())
+    if edits is not None:
+        B.set_ybus_edits(*edits)
+    stats = B.solve(max_iter=max_iter, tol=1e-8, scheduling=sched)
+    st, it, res = B.results()
+    return B.get_v(), st, it, res, stats
+
+
+def _S(g, rows, seed):
+    p, q = syn.injection_scenarios(g, rows, seed=seed)
+    return (p + 1j * q) / g.sn_mva
+
+
+# FP64 answers of two solvers differ by rounding (1e-12 of |V| = 1 after the
+# condition number of a 6,500-bus Jacobian); a mixed answer is within the
+# tolerance's distance of the root: 1e-8 pu of residual through the inverse
+# Jacobian's few tens of pu, the bound the other mixed tests use
+ATOL = {_capi.FP64: 1e-10, _capi.MIXED: 1e-7}
+
+
+@pytest.mark.parametrize("n,rows,prec", [
+    (2, 1, _capi.FP64), (3, 65, _capi.MIXED), (14, 63, _capi.FP64), (14, 130, _capi.MIXED),
+    (37, 5000, _capi.FP64), (118, 64, _capi.MIXED), (301, 700, _capi.FP64), (997, 300, _capi.FP64),
+    (2000, 1, _capi.MIXED), (2000, 300, _capi.MIXED), (2000, 70, _capi.FP64), (2000, 600, _capi.FP64),
+    (6500, 1, _capi.FP64), (6500, 300, _capi.MIXED),
+])
+def test_row_solver_matches_oracle_and_tile_kernels(n, rows, prec, monkeypatch):
+    g = _grid(n)
+    S = _S(g, rows, 41)
+    V, st, it, res, stats = _solve(g, S, prec, monkeypatch, 1)
+    Vt, stt, itt, _, stats_t = _solve(g, S, prec, monkeypatch, 0)
+    np.testing.assert_array_equal(st, stt)
+    k = min(rows, 128)
+    Vo, sto, ito, _ = orc.nr_batch(g.Ybus, g.flat_start(), S[:k], g.pv, g.pq, 10, 1e-8, n_threads=16)
+    np.testing.assert_array_equal(st[:k], sto)
+    if prec == _capi.FP64:
+        np.testing.assert_array_equal(it, itt)
+        np.testing.assert_array_equal(it[:k], ito)
+        assert stats["iterations"] == stats_t["iterations"]
+        assert stats["rows_factored"] == int(it.sum())
+    assert (st == 0).all() and (res < 1e-8).all()
+    assert np.abs(V - Vt).max() < ATOL[prec]
+    assert np.abs(V[:k] - Vo).max() < ATOL[prec]
+
+
+@pytest.mark.parametrize("prec", [_capi.FP64, _capi.MIXED])
+def test_fixed_buses(prec, monkeypatch):
+    g = _grid(118)
+    S = _S(g, 70, 42)
+    pv, pq = g.pv[3:], g.pq[5:]  # eight more buses held at their start
+    V, st, it, _, _ = _solve(g, S, prec, monkeypatch, 1, pv=pv, pq=pq)
+    Vt, stt, itt, _, _ = _solve(g, S, prec, monkeypatch, 0, pv=pv, pq=pq)
+    np.testing.assert_array_equal(st, stt)
+    assert (st == 0).all()
+    assert np.abs(V - Vt).max() < ATOL[prec]
+    held = np.concatenate([g.pv[:3], g.pq[:5], g.slack])
+    np.testing.assert_array_equal(V[:, held], np.broadcast_to(g.flat_start()[held], (70, held.size)))
+
+
+@pytest.mark.parametrize("n,prec,ir", [(118, _capi.FP64, 0), (2000, _capi.MIXED, 0), (2000, _capi.FP64, 0),
+                                       (2000, _capi.MIXED, 2), (118, _capi.MIXED, 1)])
+def test_edited_rows_and_refinement(n, prec, ir, monkeypatch):
+    g = _grid(n)
+    rows = 130
+    S = _S(g, rows, 43)
+    edits = syn.outage_edits(g, syn.random_outages(g, rows, max_k=2, seed=44))
+    V, st, it, _, _ = _solve(g, S, prec, monkeypatch, 1, edits=edits, ir=ir)
+    Vt, stt, itt, _, _ = _solve(g, S, prec, monkeypatch, 0, edits=edits, ir=ir)
+    np.testing.assert_array_equal(st, stt)
+    ok = st == 0
+    assert ok.mean() > 0.9
+    assert np.abs(V[ok] - Vt[ok]).max() < ATOL[prec]
+    if prec == _capi.FP64:
+        np.testing.assert_array_equal(it, itt)
+
+
+def test_chunked_schedule_runs_its_count(monkeypatch):
+    g = _grid(118)
+    S = _S(g, 40, 45)
+    for k in (0, 3, 6):
+        V, st, it, _, _ = _solve(g, S, _capi.FP64, monkeypatch, 1, sched=_capi.CHUNKED, max_iter=k)
+        Vt, stt, itt, _, _ = _solve(g, S, _capi.FP64, monkeypatch, 0, sched=_capi.CHUNKED, max_iter=k)
+        np.testing.assert_array_equal(st, stt)
+        np.testing.assert_array_equal(it, itt)
+        assert (it == k).all()
+        assert np.abs(V - Vt).max() < 1e-12
+
+
+@pytest.mark.parametrize("prec", [_capi.FP64, _capi.MIXED])
+def test_rows_that_do_not_converge_are_the_tile_kernels(prec, monkeypatch):
+    """Overloaded rows (no solution) among sound ones: statuses, counts, residuals
+    and voltages of the tile kernels, bit for bit."""
+    g = _grid(118)
+    S = _S(g, 150, 46)
+    hard = [3, 64, 149]
+    S[hard] *= 12.0
+    V, st, it, res, _ = _solve(g, S, prec, monkeypatch, 1)
+    Vt, stt, itt, rest, _ = _solve(g, S, prec, monkeypatch, 0)
+    np.testing.assert_array_equal(st, stt)
+    assert (st[hard] != 0).all() and (np.delete(st, hard) == 0).all()
+    np.testing.assert_array_equal(it[hard], itt[hard])
+    np.testing.assert_array_equal(res[hard], rest[hard])
+    np.testing.assert_array_equal(V[hard], Vt[hard])
+
+
+def test_learned_start_restarts(monkeypatch):
+    """A network of no use (its outputs are the flat angles plus noise) makes rows
+    restart from the fallback: restarts, statuses and voltages as the tile kernels'."""
+    from gpusim2grid_amd.warmstart import WarmStart
+    g = _grid(118)
+    rows = 200
+    S = _S(g, rows, 47)
+    rng = np.random.default_rng(7)
+    ws = WarmStart(g.n_bus, g.pv, g.pq, g.slack, np.abs(g.flat_start()), n_hidden=64, seed=3)
+    mu = np.zeros(ws.n_out, np.float32)
+    mu[1::2] = 1.0
+    ws.mlp.set_normalization(np.zeros(ws.n_in, np.float32), np.ones(ws.n_in, np.float32), mu,
+                             np.full(ws.n_out, 0.6, np.float32))
+    ws.mlp.set_params({k: rng.normal(0, 0.3, v.shape).astype(np.float32) for k, v in ws.mlp.get_params().items()})
+    out = []
+    for on in ("1", "0"):
+        monkeypatch.setenv("G2G_ROWS", on)
+        P = _capi.Plan.from_grid(g.Ybus, g.pv, g.pq, g.slack)
+        B = _capi.Batch(P, rows, precision=_capi.FP64)
+        B.set_sbus(S)
+        B.set_v(g.flat_start())
+        stats = B.solve_warm(ws.mlp, k_warm=4, growth=1.0, max_iter=10, tol=1e-8)
+        out.append((B.get_v(), *B.results(), stats))
+    (V, st, it, _, s1), (Vt, stt, itt, _, s0) = out
+    assert s1["n_requeued"] == s0["n_requeued"] > 0
+    np.testing.assert_array_equal(st, stt)
+    np.testing.assert_array_equal(it, itt)
+    assert (st == 0).all()
+    assert np.abs(V - Vt).max() < 1e-9
