@@ -857,9 +857,22 @@ struct EditLists {
 };
 
 // room for cap edits per row (the lists kept when keep is set)
+// A captured round holds the buffers' addresses: it goes before one of them
+// is replaced (the next round is captured again).
+void drop_round_graph(g2g_batch_s* b)
+{
+    if (!b->graph_exec && !b->graph) return;
+    HIPCHK(hipStreamSynchronize(b->stream));
+    if (b->graph_exec) HIPCHK(hipGraphExecDestroy(b->graph_exec));
+    b->graph_exec = nullptr;
+    if (b->graph) HIPCHK(hipGraphDestroy(b->graph));
+    b->graph = nullptr;
+}
+
 void ensure_edit_cap(g2g_batch_s* b, int cap, bool keep)
 {
     if (cap <= b->ed_cap) return;
+    drop_round_graph(b);
     cap = (cap + 7) / 8 * 8;
     const size_t n = static_cast<size_t>(b->rows_pad) * cap;
     int* ent = dalloc<int>(n);
@@ -1505,22 +1518,13 @@ void launch_row_kernel(const RowShape& s, const RowArgs<Real>& a, int grid, hipS
 
 constexpr int kRowCnt = 5;
 
-// Runs the R active rows from iteration `it` to their end; last_iter: the
-// largest iteration count.  decided: the statuses of iteration `it` already
-// stand (the mismatch there has run).  Returns the rows left as they came
-// (still active, nothing of theirs written).
+// the buffers of a launch over up to R rows
 template <typename Real>
-int solve_rows(g2g_batch_s* b, int R, int it, bool decided, int max_iter, double tol, int freeze, double growth,
-               SolveTimer& tm, long long& rows_factored, int& last_iter)
+void row_buffers(g2g_batch_s* b, const RowShape& s, int grid)
 {
-    const g2g_plan_s* P = b->plan;
-    const RowPlan& r = P->rw.r;
-    const RowShape s = row_shape<Real>(b, R);
-    hipStream_t st = b->stream;
-    const int e0 = tm.mark();
-    const int grid = std::min(R, b->n_cu * s.per_cu);
     const size_t need = s.scratch * static_cast<size_t>(grid);
     if (need > b->row_scratch_cap) {
+        drop_round_graph(b);
         dfree(b->row_scratch);
         b->row_scratch = nullptr;
         b->row_scratch_cap = 0;
@@ -1528,10 +1532,27 @@ int solve_rows(g2g_batch_s* b, int R, int it, bool decided, int max_iter, double
         b->row_scratch_cap = need;
     }
     if (!b->row_cnt) b->row_cnt = dalloc<int>(kRowCnt);
+}
+
+template <typename Real>
+int row_grid(const g2g_batch_s* b, const RowShape& s, int R)
+{
+    return std::min(R, b->n_cu * s.per_cu);
+}
+
+// The launches over R rows (listed: the active ones among more).  clock
+// (nullable), max_upd: a streamed round's iteration clock and its updates.
+template <typename Real>
+void launch_rows(g2g_batch_s* b, int R, bool listed, int it, bool decided, int max_iter, double tol, int freeze,
+                 double growth, const int* clock, int max_upd)
+{
+    const g2g_plan_s* P = b->plan;
+    const RowPlan& r = P->rw.r;
+    const RowShape s = row_shape<Real>(b, R);
+    hipStream_t st = b->stream;
+    const int grid = row_grid<Real>(b, s, R);
     k_fill_int<<<1, 64, 0, st>>>(b->row_cnt, 0, kRowCnt);
-    const bool listed = R < b->active_rows;
     if (listed) {
-        if (!b->row_list) b->row_list = dalloc<int>(static_cast<size_t>(b->rows_pad));
         k_collect_rows<<<blocks_for(b->active_rows, 256), 256, 0, st>>>(b->status, b->active_rows, b->row_list,
                                                                         b->row_cnt + 3);
         HIPCHK(hipGetLastError());
@@ -1574,6 +1595,8 @@ int solve_rows(g2g_batch_s* b, int R, int it, bool decided, int max_iter, double
     a.list_n = b->row_cnt + 3;
     a.iter0 = it;
     a.skip_first = decided ? 1 : 0;
+    a.clock = clock;
+    a.max_upd = max_upd;
     a.max_iter = max_iter;
     a.tol = tol;
     a.freeze = freeze;
@@ -1581,8 +1604,8 @@ int solve_rows(g2g_batch_s* b, int R, int it, bool decided, int max_iter, double
     a.contraction = b->contraction;
     a.pivot_eps = b->precision == G2G_MIXED ? 1e-5 : 1e-12;
     a.ir_steps = b->ir_steps;
+    if (b->streaming || b->restart_on) a.it0 = b->it0;
     if (b->restart_on) {
-        a.it0 = b->it0;
         a.budget = b->budget;
         a.warm = b->warm;
         a.V0 = b->V0;
@@ -1599,6 +1622,23 @@ int solve_rows(g2g_batch_s* b, int R, int it, bool decided, int max_iter, double
     else if (s.blk_lds) launch_row_kernel<Real, true, false>(s, a, grid, st);
     else if (s.v_lds) launch_row_kernel<Real, false, true>(s, a, grid, st);
     else launch_row_kernel<Real, false, false>(s, a, grid, st);
+}
+
+// Runs the R active rows from iteration `it` to their end; last_iter: the
+// largest iteration count.  decided: the statuses of iteration `it` already
+// stand (the mismatch there has run).  Returns the rows left as they came
+// (still active, nothing of theirs written).
+template <typename Real>
+int solve_rows(g2g_batch_s* b, int R, int it, bool decided, int max_iter, double tol, int freeze, double growth,
+               SolveTimer& tm, long long& rows_factored, int& last_iter)
+{
+    hipStream_t st = b->stream;
+    const int e0 = tm.mark();
+    const RowShape s = row_shape<Real>(b, R);
+    row_buffers<Real>(b, s, row_grid<Real>(b, s, R));
+    const bool listed = R < b->active_rows;
+    if (listed && !b->row_list) b->row_list = dalloc<int>(static_cast<size_t>(b->rows_pad));
+    launch_rows<Real>(b, R, listed, it, decided, max_iter, tol, freeze, growth, nullptr, 0);
     tm.ph[1].push_back({e0, tm.mark()});
     tm.factor_main.push_back(0);
     HIPCHK(hipMemcpyAsync(b->h_active + 4, b->row_cnt, kRowCnt * sizeof(int), hipMemcpyDeviceToHost, st));
@@ -1764,8 +1804,14 @@ int nr_loop(g2g_batch_s* b, int max_iter, double tol, int freeze, double growth,
 // last update brought it below tol is found by the next round's first
 // mismatch (its count is then the number of updates it had).
 template <typename Real>
-void stream_round_launches(g2g_batch_s* b, int k, int max_iter, double tol)
+void stream_round_launches(g2g_batch_s* b, int k, int max_iter, double tol, bool by_rows)
 {
+    if (by_rows) {  // the whole round is the row solver's
+        launch_rows<Real>(b, b->active_rows, true, 0, false, max_iter, tol, 1, 0.0, b->clock_dev, k);
+        k_add_int<<<1, 64, 0, b->stream>>>(b->clock_dev, k);
+        HIPCHK(hipGetLastError());
+        return;
+    }
     const double eps = b->precision == G2G_MIXED ? 1e-5 : 1e-12;  // own_lu/batched_lu.cuh:50-56
     for (int q = 0; q < k; ++q) {
         k_fill_int<<<1, 64, 0, b->stream>>>(b->n_active, 0, 2);
@@ -1794,9 +1840,18 @@ void stream_round(g2g_batch_s* b, int k, int max_iter, double tol)
         b->Bs = dalloc<unsigned char>(bytes);
         b->Xs = dalloc<unsigned char>(bytes);
     }
-    multiplier_stream<Real>(b);  // allocated (and cleared) outside any graph capture
+    // few slots for the grid: rounds of the row solver (its buffers, too, are
+    // allocated outside any capture)
+    const bool by_rows = k > 0 && use_rows<Real>(b, b->active_rows);
+    if (by_rows) {
+        const RowShape s = row_shape<Real>(b, b->active_rows);
+        row_buffers<Real>(b, s, row_grid<Real>(b, s, b->active_rows));
+        if (!b->row_list) b->row_list = dalloc<int>(static_cast<size_t>(b->rows_pad));
+    } else {
+        multiplier_stream<Real>(b);  // allocated (and cleared) outside any graph capture
+    }
     if (!b->stream_graph) {
-        stream_round_launches<Real>(b, k, max_iter, tol);
+        stream_round_launches<Real>(b, k, max_iter, tol, by_rows);
     } else {
         auto bits = [](double x) {
             long long v = 0;
@@ -1804,16 +1859,13 @@ void stream_round(g2g_batch_s* b, int k, int max_iter, double tol)
             return v;
         };
         // everything a round's launches take that can change between rounds
-        const long long refine = 4LL * b->ir_steps + (b->ir_fp64 ? 2 : 0) + (factor_walk_mode<Real>(b) == kFactorStoreL);
+        const long long refine = 4LL * b->ir_steps + (b->ir_fp64 ? 2 : 0) + (factor_walk_mode<Real>(b) == kFactorStoreL) + (by_rows ? 1LL << 40 : 0);
         const long long key[6] = {k, max_iter, bits(tol), refine, bits(b->max_dva), bits(b->max_dvm)};
         if (!b->graph_exec || !std::equal(key, key + 6, b->graph_key)) {
-            if (b->graph_exec) HIPCHK(hipGraphExecDestroy(b->graph_exec));
-            if (b->graph) HIPCHK(hipGraphDestroy(b->graph));
-            b->graph_exec = nullptr;
-            b->graph = nullptr;
+            drop_round_graph(b);
             // function attributes (dynamic LDS) are set by an eager round
             // first, so the capture records kernel launches only
-            stream_round_launches<Real>(b, k, max_iter, tol);
+            stream_round_launches<Real>(b, k, max_iter, tol, by_rows);
             b->clock += k;
             if (!b->graph_stream) {
                 if (b->stream) {
@@ -1828,7 +1880,7 @@ void stream_round(g2g_batch_s* b, int k, int max_iter, double tol)
             b->stream = b->graph_stream;  // the launches below are recorded on it
             HIPCHK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeRelaxed));
             try {
-                stream_round_launches<Real>(b, k, max_iter, tol);
+                stream_round_launches<Real>(b, k, max_iter, tol, by_rows);
             } catch (...) {
                 hipGraph_t g = nullptr;
                 (void)hipStreamEndCapture(b->stream, &g);

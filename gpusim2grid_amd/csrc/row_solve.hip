@@ -230,7 +230,7 @@ __global__ __launch_bounds__(kRowMaxThreads) void k_row_solve(RowArgs<Real> a)
         double prev = a.res[row];
         double growth = a.growth;
         bool decide = !a.skip_first;
-        int iter = a.iter0, st = kActive, n_upd = 0;
+        int iter = a.clock ? *a.clock + a.iter0 : a.iter0, st = kActive, n_upd = 0;
         double jm = 0.0;
         if (tid == 0) *slice_next = n_wave;
         __syncthreads();
@@ -504,7 +504,7 @@ __global__ __launch_bounds__(kRowMaxThreads) void k_row_solve(RowArgs<Real> a)
                 __syncthreads();
                 continue;
             }
-            if (st != kActive || iter >= a.max_iter) break;
+            if (st != kActive || it >= a.max_iter) break;
             growth = a.growth;
             decide = true;
             const Real eps = static_cast<Real>(a.pivot_eps) * static_cast<Real>(jm);
@@ -571,8 +571,9 @@ __global__ __launch_bounds__(kRowMaxThreads) void k_row_solve(RowArgs<Real> a)
             ++iter;
             ++n_upd;
             __syncthreads();
+            if (a.max_upd > 0 && n_upd >= a.max_upd) break;  // st: still active
         }
-        if (st != kConverged && !(prev < kRowKeep)) {
+        if (!a.clock && st != kConverged && !(prev < kRowKeep)) {
             if (tid == 0) atomicAdd(a.left, 1);
             continue;
         }

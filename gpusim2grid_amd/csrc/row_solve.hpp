@@ -12,7 +12,8 @@ constexpr int kRowMaxThreads = 1024;
 // A row that ends unconverged with a residual above this (or not finite) is
 // left as it came, for the tile kernels to finish: the iterates of a row that
 // does not contract amplify rounding, so its last one is the solver's own, and
-// callers keep getting the one they always got.
+// callers keep getting the one they always got.  (Not in streamed rounds, where
+// a row's V moves on with every launch.)
 constexpr double kRowKeep = 1e-4;
 
 template <typename Real>
@@ -46,6 +47,8 @@ struct RowArgs {
     const int* list;        // nullable: the active rows; count at list_n
     const int* list_n;
     int iter0, skip_first;  // first iteration; 1: its statuses are already decided
+    const int* clock;       // nullable: the first iteration is *clock + iter0 (streamed rounds)
+    int max_upd;            // > 0: updates of one launch (a row not ended then stays active)
     int max_iter;
     double tol;
     int freeze;

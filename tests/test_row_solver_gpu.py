@@ -168,3 +168,48 @@ def test_learned_start_restarts(monkeypatch):
     np.testing.assert_array_equal(it, itt)
     assert (st == 0).all()
     assert np.abs(V - Vt).max() < 1e-9
+
+
+@pytest.mark.parametrize("n,prec", [(118, _capi.FP64), (2000, _capi.MIXED)])
+def test_streamed_rounds(n, prec, monkeypatch):
+    """Slots filled in two goes, rounds of one and three updates (graph replays
+    among them), a scratch and an edit-list capacity that grow between rounds:
+    the same answers as a plain solve of the tile kernels."""
+    g = _grid(n)
+    rows = 150
+    S = _S(g, rows, 48)
+    outs = syn.random_outages(g, rows, max_k=2, seed=49)
+    edits = syn.outage_edits(g, outs)
+    Vt, stt, itt, _, _ = _solve(g, S, prec, monkeypatch, 0, edits=edits)
+    monkeypatch.setenv("G2G_ROWS", "1")
+    P = _capi.Plan.from_grid(g.Ybus, g.pv, g.pq, g.slack)
+    B = _capi.Batch(P, rows, precision=prec, per_row_ybus=True)
+
+    def part(r0, r1):
+        rp, en, de = edits
+        return rp[r0:r1 + 1] - rp[r0], en[rp[r0]:rp[r1]], de[rp[r0]:rp[r1]]
+
+    for go in range(2):
+        B.stream_begin()
+        B.stream_fill(np.arange(100), S[:100], g.flat_start()[None], edits=part(0, 100))
+        for _ in range(3):
+            B.stream_round(k=1, max_iter=10, tol=1e-8)
+        if go == 1:  # twenty edits on one row (entries repeated and undone): the lists grow
+            rp, en, de = part(100, 101)
+            k = np.arange(20) % g.Ybus.nnz
+            z = (np.array([0, en.size + 20], np.int32), np.concatenate([en, k]), np.concatenate([de, np.zeros(20)]))
+            B.stream_fill([100], S[100:101], g.flat_start()[None], edits=z)
+            B.stream_fill(np.arange(101, rows), S[101:], g.flat_start()[None], edits=part(101, rows))
+        else:
+            B.stream_fill(np.arange(100, rows), S[100:], g.flat_start()[None], edits=part(100, rows))
+        for _ in range(12):
+            B.stream_round(k=1 if go else 3, max_iter=10, tol=1e-8)
+            st, it, _ = B.results()
+            if not (st == -1).any():
+                break
+        np.testing.assert_array_equal(st, stt)
+        if prec == _capi.FP64:
+            np.testing.assert_array_equal(it, itt)
+        V = B.stream_take(np.arange(rows))
+        ok = st == 0
+        assert np.abs(V[ok] - Vt[ok]).max() < ATOL[prec]
