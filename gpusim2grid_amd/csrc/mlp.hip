@@ -3,12 +3,11 @@
 // A 3-layer MLP (in -> hidden -> hidden -> out, GELU) maps a row's per-bus
 // injections (and outage mask) to its voltage angles and magnitudes.  Every
 // product runs on the bf16 matrix cores with fp32 accumulation
-// (v_mfma_f32_32x32x16_bf16): one tiled GEMM kernel, templated on the operand
-// layouts (each operand row- or column-major, which covers the forward
-// X W, the backward dY W^T and the weight gradient X^T dY) and on a fused
-// epilogue (bias + GELU with the pre-activation kept for the backward pass,
-// bias only, GELU derivative).  Weights are kept in fp32 (Adam state) with a
-// bf16 copy the GEMMs read.
+// (v_mfma_f32_32x32x16_bf16) in one form, C = A B^T with both operands
+// K-contiguous: whoever writes an activation, a gradient or a weight writes
+// the transpose that the other products read beside it, into rows padded to 8
+// (zeros), so no product transposes on the way in and any width takes the
+// wide loads.  Weights are fp32 (Adam state) with bf16 copies the products read.
 //
 // The gpusim2grid reference has no learned component; this follows the
 // model the reference's paper benchmarks time as "PFdelta" MLPs
@@ -85,9 +84,10 @@ __device__ __forceinline__ void load_tiles(const GemmArgs& g, int m0, int n0, in
     }
 }
 
-// C = A B, 128 x 128 output tile per workgroup of 4 waves (each 64 x 64 as
+// C = op(A) op(B) of any layout and alignment (the product entry point's
+// general case): 128 x 128 output tile per workgroup of 4 waves (each 64 x 64 as
 // 2 x 2 MFMA 32 x 32 tiles), K in steps of 32 through LDS.
-template <bool TA, bool TB, int EPI>
+template <bool TA, bool TB>
 __global__ __launch_bounds__(256) void k_gemm(GemmArgs g)
 {
     __shared__ __align__(16) __bf16 sA[kBM][kPadK];
@@ -124,7 +124,7 @@ __global__ __launch_bounds__(256) void k_gemm(GemmArgs g)
         }
         __syncthreads();
     }
-    // epilogue: lane holds column lane % 32 and rows 8 (r / 4) + 4 (lane / 32) + r % 4
+    // lane holds column lane % 32 and rows 8 (r / 4) + 4 (lane / 32) + r % 4
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -133,31 +133,85 @@ __global__ __launch_bounds__(256) void k_gemm(GemmArgs g)
             for (int r = 0; r < 16; ++r) {
                 const int m = m0 + wm * 64 + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
                 const int n = n0 + wn * 64 + j * 32 + lr;
-                if (m >= g.M || n >= g.N) continue;
-                const float v = acc[i][j][r];
-                const long long mc = static_cast<long long>(m);
-                if (EPI == kEpiF32) {
-                    g.C[mc * g.ldc + n] = v;
-                } else if (EPI == kEpiBiasF32) {
-                    g.C[mc * g.ldc + n] = v + g.bias[n];
-                } else if (EPI == kEpiBiasGeluBf16) {
-                    const float z = v + g.bias[n];
-                    g.Z[mc * g.ldz + n] = z;
-                    g.H[mc * g.ldh + n] = static_cast<__bf16>(gelu(z));
-                } else {  // kEpiGeluBwd: dZ = (dH) * gelu'(Z), fp32 and bf16
-                    const float dz = v * gelu_grad(g.Z[mc * g.ldz + n]);
-                    g.C[mc * g.ldc + n] = dz;
-                    g.H[mc * g.ldh + n] = static_cast<__bf16>(dz);
-                }
+                if (m < g.M && n < g.N) g.C[static_cast<long long>(m) * g.ldc + n] = acc[i][j][r];
             }
 }
 
-// Forward GEMM with both operands K-contiguous: C = A Bt^T, A: M x K (row
-// m at A + m lda), Bt: N x K (row n at B + n ldb), K a multiple of 8 and rows
-// 16-byte aligned.  128 x 128 output tile per workgroup of 4 waves (each
-// 64 x 64 as 2 x 2 MFMA 32x32x16 tiles); K in steps of 64 through a
-// double-buffered LDS stage, the next step's global loads in flight while
-// the current one is multiplied.
+// One 32 x 32 block of a product at (mb, nb): lane holds column lane % 32 and
+// rows 8 (r / 4) + 4 (lane / 32) + r % 4, so four consecutive rows of a column,
+// one 8-byte store of the transpose.  sq collects the lane's sum of squares.
+template <int EPI>
+__device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, int mb, int nb, const f32x16& v, float& sq)
+{
+    const int lane = threadIdx.x & 63;
+    const int n = nb + (lane & 31), m0 = mb + 4 * (lane >> 5);
+    const bool cols = n < g.N;
+    float col = 0.0f;
+    const float bias = (EPI == kEpiBiasF32 || EPI == kEpiGelu || EPI == kEpiMse) && cols ? g.bias[n] : 0.0f;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int mq = m0 + 8 * q;
+        __bf16 h[4];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const int m = mq + s;
+            const bool in = cols && m < g.M;
+            const long long mc = m;
+            const float x = v[4 * q + s];
+            float y = 0.0f;
+            if (EPI == kEpiF32) {
+                if (in) g.C[mc * g.ldc + n] = x;
+            } else if (EPI == kEpiBiasF32) {
+                if (in) g.C[mc * g.ldc + n] = x + bias;
+            } else if (EPI == kEpiGrad) {
+                if (in) {
+                    g.C[mc * g.ldc + n] = x;
+                    sq = fmaf(x, x, sq);
+                }
+            } else if (EPI == kEpiGelu) {
+                const float z = x + bias;
+                if (in && g.Z) g.Z[mc * g.ldz + n] = z;
+                y = in ? gelu(z) : 0.0f;
+            } else if (EPI == kEpiGeluBwd) {
+                y = in ? x * gelu_grad(g.Z[mc * g.ldz + n]) : 0.0f;
+                col += y;
+            } else {  // kEpiMse
+                const float d = in ? x + bias - g.T[mc * g.ldc + n] : 0.0f;
+                sq = fmaf(d, d, sq);
+                y = 2.0f * g.scale * d;
+                col += y;
+            }
+            if (EPI == kEpiGelu || EPI == kEpiGeluBwd || EPI == kEpiMse) {
+                h[s] = static_cast<__bf16>(y);
+                if (in && g.H) g.H[mc * g.ldh + n] = h[s];
+            }
+        }
+        if (EPI == kEpiGelu || EPI == kEpiGeluBwd || EPI == kEpiMse) {
+            if (g.Ht && cols && mq < g.Mt) {
+                uint2 w;
+                __builtin_memcpy(&w, h, sizeof(w));
+                *reinterpret_cast<uint2*>(g.Ht + static_cast<long long>(n) * g.Mt + mq) = w;
+            }
+        }
+    }
+    if (EPI == kEpiGeluBwd || EPI == kEpiMse) {
+        col += __shfl_xor(col, 32, 64);
+        if (lane < 32 && cols && mb < g.M) g.colsum[static_cast<long long>(mb / 32) * g.N + n] = col;
+    }
+}
+
+__device__ __forceinline__ float wave_sum(float x)
+{
+    for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
+    return x;
+}
+
+// C = A B^T: 128 x 128 output tile per workgroup of 4 waves (each 64 x 64 as
+// 2 x 2 MFMA 32x32x16 tiles); K in steps of 64 through a double-buffered LDS
+// stage, the next step's global loads in flight while the current one is
+// multiplied.  A product with few tiles and a long K (512 x 1,024 outputs over
+// 13,000 inputs: 32 tiles) is split over gridDim.z, the partial sums added in
+// split order by k_gemm_sum (unsplit on 32 of 256 CUs: about 270 us; split by 8: 45 + 9 us).
 constexpr int kFK = 64, kFPad = 8;
 
 __device__ __forceinline__ void kc_load(const __bf16* base, long long ld, int rows, int r0, int k0, int K, int t,
@@ -199,17 +253,23 @@ __global__ __launch_bounds__(256) void k_gemm_kc(GemmArgs g)
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
     const int lr = lane & 31, lk = (lane >> 5) * 8;
     u32x4 ra[4], rb[4];
-    kc_load(g.A, g.lda, g.M, m0, 0, g.K, t, ra);
-    kc_load(g.B, g.ldb, g.N, n0, 0, g.K, t, rb);
+    int kb = 0, ke = g.K;
+    if (EPI == kEpiF32 && g.k_split > 0) {
+        kb = static_cast<int>(blockIdx.z) * g.k_split;
+        ke = min(kb + g.k_split, g.K);
+        g.C += static_cast<long long>(blockIdx.z) * g.M * g.N;
+    }
+    kc_load(g.A, g.lda, g.M, m0, kb, ke, t, ra);
+    kc_load(g.B, g.ldb, g.N, n0, kb, ke, t, rb);
     kc_store(sA[0], t, ra);
     kc_store(sB[0], t, rb);
     __syncthreads();
     int cur = 0;
-    for (int k0 = 0; k0 < g.K; k0 += kFK) {
-        const bool more = k0 + kFK < g.K;
+    for (int k0 = kb; k0 < ke; k0 += kFK) {
+        const bool more = k0 + kFK < ke;
         if (more) {
-            kc_load(g.A, g.lda, g.M, m0, k0 + kFK, g.K, t, ra);
-            kc_load(g.B, g.ldb, g.N, n0, k0 + kFK, g.K, t, rb);
+            kc_load(g.A, g.lda, g.M, m0, k0 + kFK, ke, t, ra);
+            kc_load(g.B, g.ldb, g.N, n0, k0 + kFK, ke, t, rb);
         }
 #pragma unroll
         for (int kk = 0; kk < kFK; kk += 16) {
@@ -233,130 +293,247 @@ __global__ __launch_bounds__(256) void k_gemm_kc(GemmArgs g)
         __syncthreads();
         cur ^= 1;
     }
+    float sq = 0.0f;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int j = 0; j < 2; ++j)
+            gemm_epilogue<EPI>(g, m0 + wm * 64 + i * 32, n0 + wn * 64 + j * 32, acc[i][j], sq);
+    if (EPI == kEpiGrad || EPI == kEpiMse) {
+        sq = wave_sum(sq);
+        if (lane == 0) g.sums[(blockIdx.y * gridDim.x + blockIdx.x) * 4 + wave] = sq;
+    }
+}
+
+// a split product's sum and epilogue: one wave per 32 x 32 outputs (a split
+// product has few of them, so one per workgroup)
+template <int EPI>
+__global__ __launch_bounds__(64) void k_gemm_sum(GemmArgs g, const float* __restrict__ part, int splits)
+{
+    const int lane = threadIdx.x;
+    const int mb = blockIdx.y * 32, nb = blockIdx.x * 32;
+    const int n = nb + (lane & 31);
+    const long long mn = static_cast<long long>(g.M) * g.N;
+    // every output's split is loaded before any is added: 16 loads in flight
+    f32x16 v;
+    long long at[16];
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int m = m0 + wm * 64 + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                const int n = n0 + wn * 64 + j * 32 + lr;
-                if (m >= g.M || n >= g.N) continue;
-                const float v = acc[i][j][r];
-                const long long mc = static_cast<long long>(m);
-                if (EPI == kEpiF32) {
-                    g.C[mc * g.ldc + n] = v;
-                } else if (EPI == kEpiBiasF32) {
-                    g.C[mc * g.ldc + n] = v + g.bias[n];
-                } else if (EPI == kEpiBiasGeluBf16) {
-                    const float z = v + g.bias[n];
-                    if (g.Z) g.Z[mc * g.ldz + n] = z;
-                    g.H[mc * g.ldh + n] = static_cast<__bf16>(gelu(z));
-                }
+    for (int r = 0; r < 16; ++r) {
+        const int m = mb + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+        at[r] = static_cast<long long>(m < g.M ? m : 0) * g.N + (n < g.N ? n : 0);
+        v[r] = part[at[r]];
+    }
+    for (int s = 1; s < splits; ++s) {
+        const float* p = part + s * mn;
+        float x[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) x[r] = p[at[r]];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) v[r] += x[r];
+    }
+    float sq = 0.0f;
+    gemm_epilogue<EPI>(g, mb, nb, v, sq);
+    if (EPI == kEpiGrad || EPI == kEpiMse) {
+        sq = wave_sum(sq);
+        if (lane == 0) g.sums[blockIdx.y * gridDim.x + blockIdx.x] = sq;
+    }
+}
+
+// a 64 x 64 bf16 tile in LDS: [k][n], written out as rows n of 64 consecutive k
+constexpr int kTT = 64, kTPitch = kTT + 2;
+__device__ __forceinline__ void store_transposed(const __bf16 (*tile)[kTPitch], int k0, int n0, int K, int N,
+                                                 __bf16* Wt, long long ldt)
+{
+    // 16-byte chunks of 8 k; rows are padded to a multiple of 8 (the tile holds zeros past K)
+    for (int c = threadIdx.x; c < kTT * kTT / 8; c += 256) {
+        const int n = c / (kTT / 8), k = (c % (kTT / 8)) * 8;
+        if (n0 + n >= N || k0 + k >= (K + 7) / 8 * 8) continue;
+        __bf16 h[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) h[i] = tile[k + i][n];
+        u32x4 w;
+        __builtin_memcpy(&w, h, sizeof(w));
+        *reinterpret_cast<u32x4*>(Wt + static_cast<long long>(n0 + n) * ldt + k0 + k) = w;
+    }
+}
+
+__device__ __forceinline__ float adam(float& w, float& m, float& v, float g, const AdamArgs& a, float gs)
+{
+    const float gi = g * gs;
+    const float mi = a.b1 * m + (1.0f - a.b1) * gi;
+    const float vi = a.b2 * v + (1.0f - a.b2) * gi * gi;
+    m = mi;
+    v = vi;
+    w = w - a.lr * (mi * a.c1) / (sqrtf(vi * a.c2) + a.eps);
+    return w;
+}
+
+// min(1, clip / ||g||)
+__device__ __forceinline__ float grad_scale(const AdamArgs& a)
+{
+    if (!a.gnorm2) return 1.0f;
+    const float nrm = sqrtf(*a.gnorm2);
+    return nrm > a.clip ? a.clip / nrm : 1.0f;
+}
+
+// Bound by HBM: 28 bytes a weight of fp32 state and 2 - 4 of copies; the
+// transposed copy goes through LDS here instead of a pass of its own that
+// reads the weights again (59 us of a 6,500-bus step).
+__global__ __launch_bounds__(256) void k_weights(float* __restrict__ w, float* __restrict__ m, float* __restrict__ v,
+                                                 const float* __restrict__ g, int K, int N, AdamArgs a,
+                                                 __bf16* __restrict__ Wt, long long ldt, __bf16* __restrict__ Wn,
+                                                 long long ldn)
+{
+    __shared__ __bf16 tile[kTT][kTPitch];
+    const int k0 = blockIdx.y * kTT, n0 = blockIdx.x * kTT;
+    const int c = (threadIdx.x & 15) * 4, r = threadIdx.x >> 4;
+    const float gs = m ? grad_scale(a) : 1.0f;
+    const bool wide = (N & 3) == 0;  // rows and matrices start 16-byte aligned
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int k = k0 + r + 16 * i, n = n0 + c;
+        float x[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        const long long at = static_cast<long long>(k) * N + n;
+        if (k < K && wide && n < N) {
+            float4 w4 = *reinterpret_cast<const float4*>(w + at);
+            if (m) {
+                float4 m4 = *reinterpret_cast<const float4*>(m + at), v4 = *reinterpret_cast<const float4*>(v + at);
+                const float4 g4 = *reinterpret_cast<const float4*>(g + at);
+                adam(w4.x, m4.x, v4.x, g4.x, a, gs);
+                adam(w4.y, m4.y, v4.y, g4.y, a, gs);
+                adam(w4.z, m4.z, v4.z, g4.z, a, gs);
+                adam(w4.w, m4.w, v4.w, g4.w, a, gs);
+                *reinterpret_cast<float4*>(w + at) = w4;
+                *reinterpret_cast<float4*>(m + at) = m4;
+                *reinterpret_cast<float4*>(v + at) = v4;
             }
-}
-
-// Wt (N x K, bf16) = transpose of W (K x N, fp32), 32 x 32 tiles through LDS
-__global__ void k_transpose_bf16(const float* __restrict__ W, int K, int N, __bf16* __restrict__ Wt)
-{
-    __shared__ float tile[32][33];
-    const int k0 = blockIdx.y * 32, n0 = blockIdx.x * 32;
-    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;  // 256 threads: 32 x 8
-    for (int r = ty; r < 32; r += 8) {
-        const int k = k0 + r, n = n0 + tx;
-        tile[r][tx] = (k < K && n < N) ? W[static_cast<long long>(k) * N + n] : 0.0f;
+            x[0] = w4.x;
+            x[1] = w4.y;
+            x[2] = w4.z;
+            x[3] = w4.w;
+        } else if (k < K) {
+            for (int j = 0; j < 4 && n + j < N; ++j) {
+                float wj = w[at + j];
+                if (m) {
+                    float mj = m[at + j], vj = v[at + j];
+                    adam(wj, mj, vj, g[at + j], a, gs);
+                    w[at + j] = wj;
+                    m[at + j] = mj;
+                    v[at + j] = vj;
+                }
+                x[j] = wj;
+            }
+        }
+        __bf16 h[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            h[j] = static_cast<__bf16>(x[j]);
+            tile[r + 16 * i][c + j] = h[j];
+        }
+        if (Wn && k < K && n < ldn) {  // (ldn a multiple of 8: pads get their zeros)
+            uint2 p;
+            __builtin_memcpy(&p, h, sizeof(p));
+            *reinterpret_cast<uint2*>(Wn + static_cast<long long>(k) * ldn + n) = p;
+        }
     }
     __syncthreads();
-    for (int r = ty; r < 32; r += 8) {
-        const int n = n0 + r, k = k0 + tx;
-        if (n < N && k < K) Wt[static_cast<long long>(n) * K + k] = static_cast<__bf16>(tile[tx][r]);
+    store_transposed(tile, k0, n0, K, N, Wt, ldt);
+}
+
+__global__ __launch_bounds__(256) void k_adam_bias(float* __restrict__ w, float* __restrict__ m,
+                                                   float* __restrict__ v, const float* __restrict__ g, BiasSegs s,
+                                                   AdamArgs a)
+{
+    int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const float gs = grad_scale(a);
+    for (int q = 0; q < 3; ++q) {
+        if (i < s.len[q]) {
+            const long long at = s.off[q] + i;
+            adam(w[at], m[at], v[at], g[at], a, gs);
+            return;
+        }
+        i -= s.len[q];
     }
 }
 
-// column sums of an fp32 M x N matrix (bias gradients), one thread per column
-// Column sums of X [M][N] accumulated into out (zeroed by the caller): a
-// block sums kColRows rows of 64 columns, four row groups per column reduced
-// in LDS, then one atomic per column.  Grid: (ceil(N / 64), ceil(M / kColRows)).
-__global__ __launch_bounds__(256) void k_colsum(const float* __restrict__ X, long long ldx, int M, int N,
-                                                float* __restrict__ out)
-{
-    __shared__ float part[4][64];
-    const int c = threadIdx.x & 63, g = threadIdx.x >> 6;
-    const int n = blockIdx.x * 64 + c;
-    const int m0 = blockIdx.y * kColRows;
-    const int m1 = m0 + kColRows < M ? m0 + kColRows : M;
-    float s = 0.0f;
-    if (n < N)
-        for (int m = m0 + g; m < m1; m += 4) s += X[static_cast<long long>(m) * ldx + n];
-    part[g][c] = s;
-    __syncthreads();
-    if (g == 0 && n < N) atomicAdd(&out[n], part[0][c] + part[1][c] + part[2][c] + part[3][c]);
-}
-
-// MSE loss gradient dY = 2 (Y - T) / (M N) (fp32 and bf16) and the loss sum:
-// grid-stride over the elements, one atomic per block
-__global__ __launch_bounds__(256) void k_mse_grad(const float* __restrict__ Y, const float* __restrict__ T,
-                                                  long long n_el, float scale, float* __restrict__ dY,
-                                                  __bf16* __restrict__ dYb, float* __restrict__ loss)
+__global__ __launch_bounds__(256) void k_bias_grad(BiasGradArgs a)
 {
     __shared__ float part[4];
-    float e = 0.0f;
-    for (long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x; i < n_el;
-         i += static_cast<long long>(gridDim.x) * blockDim.x) {
-        const float d = Y[i] - T[i];
-        e += d * d;
-        dY[i] = 2.0f * scale * d;
-        dYb[i] = static_cast<__bf16>(2.0f * scale * d);
+    int i = blockIdx.x * blockDim.x + threadIdx.x;
+    float x = 0.0f;
+    for (int q = 0; q < 3; ++q) {
+        if (i >= 0 && i < a.s.len[q]) {
+            for (int r = 0; r < a.rows; ++r) x += a.colsum[q][static_cast<long long>(r) * a.s.len[q] + i];
+            a.g[a.s.off[q] + i] = x;
+        }
+        i -= a.s.len[q];
     }
-    for (int o = 32; o > 0; o >>= 1) e += __shfl_down(e, o, 64);
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = e;
+    const float sq = wave_sum(x * x);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = sq;
     __syncthreads();
-    if (threadIdx.x == 0) atomicAdd(loss, (part[0] + part[1] + part[2] + part[3]) * scale);
+    if (threadIdx.x == 0) a.sums[blockIdx.x] = part[0] + part[1] + part[2] + part[3];
 }
 
-// sum of squares of x[0..n) added into *out (the gradient's norm for clipping)
-__global__ __launch_bounds__(256) void k_sumsq(const float* __restrict__ x, long long n, float* __restrict__ out)
+__global__ __launch_bounds__(1024) void k_finish(const float* __restrict__ a, int na, float scale,
+                                                 const float* __restrict__ b, int nb, float* __restrict__ loss,
+                                                 float* __restrict__ gnorm2)
 {
-    __shared__ float s[256];
-    float a = 0.0f;
-    for (long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
-         i += static_cast<long long>(gridDim.x) * blockDim.x)
-        a = fmaf(x[i], x[i], a);
-    s[threadIdx.x] = a;
+    __shared__ float sa[16], sb[16];
+    float x = 0.0f, y = 0.0f;
+    for (int i = threadIdx.x; i < na; i += 1024) x += a[i];
+    for (int i = threadIdx.x; i < nb; i += 1024) y += b[i];
+    x = wave_sum(x);
+    y = wave_sum(y);
+    if ((threadIdx.x & 63) == 0) {
+        sa[threadIdx.x >> 6] = x;
+        sb[threadIdx.x >> 6] = y;
+    }
     __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (static_cast<int>(threadIdx.x) < w) s[threadIdx.x] += s[threadIdx.x + w];
-        __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int i = 1; i < 16; ++i) {
+            x += sa[i];
+            y += sb[i];
+        }
+        *loss = scale * x;
+        *gnorm2 = y;
     }
-    if (threadIdx.x == 0) atomicAdd(out, s[0]);
 }
 
-// Adam on fp32 master weights, refreshing the bf16 copy (nullable).  With
-// gnorm2 (nullable) the gradient is scaled by min(1, clip / ||g||) first.
-__global__ void k_adam(float* __restrict__ w, float* __restrict__ m, float* __restrict__ v,
-                       const float* __restrict__ g, long long n, float lr, float b1, float b2, float eps,
-                       float c1, float c2, __bf16* __restrict__ wb, const float* __restrict__ gnorm2, float clip)
+__global__ __launch_bounds__(256) void k_stage_x(const float* __restrict__ X, int M, int n, __bf16* __restrict__ Xb,
+                                                 long long ldx, __bf16* __restrict__ Xt, int Mt)
 {
-    const long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    float gi = g[i];
-    if (gnorm2) {
-        const float nrm = sqrtf(*gnorm2);
-        if (nrm > clip) gi *= clip / nrm;
+    __shared__ __bf16 tile[kTT][kTPitch];
+    const int m0 = blockIdx.y * kTT, n0 = blockIdx.x * kTT;
+    const int c = (threadIdx.x & 15) * 4, r = threadIdx.x >> 4;
+    const bool wide = (n & 3) == 0 && (reinterpret_cast<uintptr_t>(X) & 15) == 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int m = m0 + r + 16 * i, k = n0 + c;
+        float x[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (m < M && wide && k < n) {
+            const float4 q = *reinterpret_cast<const float4*>(X + static_cast<long long>(m) * n + k);
+            x[0] = q.x;
+            x[1] = q.y;
+            x[2] = q.z;
+            x[3] = q.w;
+        } else if (m < M) {
+            for (int j = 0; j < 4 && k + j < n; ++j) x[j] = X[static_cast<long long>(m) * n + k + j];
+        }
+        __bf16 h[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            h[j] = static_cast<__bf16>(x[j]);
+            tile[r + 16 * i][c + j] = h[j];
+        }
+        if (m < M && k < ldx) {
+            uint2 p;
+            __builtin_memcpy(&p, h, sizeof(p));
+            *reinterpret_cast<uint2*>(Xb + static_cast<long long>(m) * ldx + k) = p;
+        }
     }
-    const float mi = b1 * m[i] + (1.0f - b1) * gi;
-    const float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
-    m[i] = mi;
-    v[i] = vi;
-    const float wi = w[i] - lr * (mi * c1) / (sqrtf(vi * c2) + eps);
-    w[i] = wi;
-    if (wb) wb[i] = static_cast<__bf16>(wi);
-}
-
-__global__ void k_f32_to_bf16(const float* __restrict__ x, long long n, __bf16* __restrict__ y)
-{
-    const long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < n) y[i] = static_cast<__bf16>(x[i]);
+    if (!Xt) return;
+    __syncthreads();
+    store_transposed(tile, m0, n0, M, n, Xt, Mt);
 }
 
 // Features and start voltages in the batch's tiled layout, [row / 64][bus][row % 64]:
@@ -477,13 +654,18 @@ __global__ __launch_bounds__(256) void k_warm_v_tiles_t(const float* __restrict_
 
 template __global__ void k_gemm_kc<kEpiF32>(GemmArgs);
 template __global__ void k_gemm_kc<kEpiBiasF32>(GemmArgs);
-template __global__ void k_gemm_kc<kEpiBiasGeluBf16>(GemmArgs);
-template __global__ void k_gemm<false, false, kEpiF32>(GemmArgs);
-template __global__ void k_gemm<false, false, kEpiBiasF32>(GemmArgs);
-template __global__ void k_gemm<false, false, kEpiBiasGeluBf16>(GemmArgs);
-template __global__ void k_gemm<false, true, kEpiF32>(GemmArgs);
-template __global__ void k_gemm<false, true, kEpiGeluBwd>(GemmArgs);
-template __global__ void k_gemm<true, false, kEpiF32>(GemmArgs);
-template __global__ void k_gemm<true, true, kEpiF32>(GemmArgs);
+template __global__ void k_gemm_kc<kEpiGelu>(GemmArgs);
+template __global__ void k_gemm_kc<kEpiGeluBwd>(GemmArgs);
+template __global__ void k_gemm_kc<kEpiMse>(GemmArgs);
+template __global__ void k_gemm_kc<kEpiGrad>(GemmArgs);
+template __global__ void k_gemm_sum<kEpiBiasF32>(GemmArgs, const float*, int);
+template __global__ void k_gemm_sum<kEpiGelu>(GemmArgs, const float*, int);
+template __global__ void k_gemm_sum<kEpiGeluBwd>(GemmArgs, const float*, int);
+template __global__ void k_gemm_sum<kEpiMse>(GemmArgs, const float*, int);
+template __global__ void k_gemm_sum<kEpiGrad>(GemmArgs, const float*, int);
+template __global__ void k_gemm<false, false>(GemmArgs);
+template __global__ void k_gemm<false, true>(GemmArgs);
+template __global__ void k_gemm<true, false>(GemmArgs);
+template __global__ void k_gemm<true, true>(GemmArgs);
 
 }  // namespace g2g

@@ -26,9 +26,10 @@ struct g2g_mlp_s {
     float* m = nullptr;
     float* v = nullptr;
     float* g = nullptr;
-    __bf16* wb = nullptr;  // bf16 copy of all parameters (the GEMMs read the weight parts)
-    __bf16* wt = nullptr;  // bf16 transposed weights (N x K) for the K-contiguous forward GEMM
-    bool kc = false;       // every width a multiple of 8: the forward uses k_gemm_kc
+    // bf16 copies the products read, rows K-contiguous and padded to 8: the
+    // transposed weights (forward) and, of the upper layers, the weights as
+    // they are (backward)
+    __bf16 *W1t = nullptr, *W2t = nullptr, *W3t = nullptr, *W2n = nullptr, *W3n = nullptr;
     int step = 0;
     // normalisation (features: z-score per input; outputs: per output)
     float* in_mu = nullptr;
@@ -39,45 +40,46 @@ struct g2g_mlp_s {
     int* kind = nullptr;
     double* vfix = nullptr;
     int n_bus = 0;
-    // workspace for M rows
+    // workspace of M rows: activations (rows padded to 8) ...
     int ws_M = 0;
-    __bf16* X = nullptr;
-    float* Z1 = nullptr;
-    float* Z2 = nullptr;
-    __bf16* H1 = nullptr;
-    __bf16* H2 = nullptr;
+    __bf16 *X = nullptr, *H1 = nullptr, *H2 = nullptr;
     float* Y = nullptr;
-    float* T = nullptr;
-    float* dY = nullptr;
-    __bf16* dYb = nullptr;
-    float* dZ1 = nullptr;
-    float* dZ2 = nullptr;
-    __bf16* dZ1b = nullptr;
-    __bf16* dZ2b = nullptr;
+    // ... and of a training step: pre-activations, transposes (rows of M
+    // padded to 8), gradients, column sums of 32 rows, sums of squares
+    int tr_M = 0;
+    float *Z1 = nullptr, *Z2 = nullptr, *T = nullptr;
+    __bf16 *Xt = nullptr, *H1t = nullptr, *H2t = nullptr, *dYb = nullptr, *dYt = nullptr, *dZ2b = nullptr, *dZ2t = nullptr,
+           *dZ1t = nullptr;
+    float *cs1 = nullptr, *cs2 = nullptr, *cs3 = nullptr, *sums = nullptr, *loss_sums = nullptr;
+    // partial sums of split products (grown on use)
+    float* part = nullptr;
+    size_t part_cap = 0;
     float* loss = nullptr;
     float clip = 0.0f;          // gradient-norm clip of the training steps (0: off)
-    float* gnorm2 = nullptr;    // its squared-norm accumulator
-    DeviceScratch ws;   // workspace buffers (freed on growth / destruction)
-    DeviceScratch own;  // parameters and state
+    DeviceScratch ws, tr, pt;  // workspace buffers (freed on growth / destruction)
+    DeviceScratch own;         // parameters and state
 
-    __bf16* W1b() const { return wb + o_W1; }
-    __bf16* W2b() const { return wb + o_W2; }
-    __bf16* W3b() const { return wb + o_W3; }
-    __bf16* W1t() const { return wt + o_W1; }
-    __bf16* W2t() const { return wt + o_W2; }
-    __bf16* W3t() const { return wt + o_W3; }
+    static int pad8(int n) { return (n + 7) / 8 * 8; }
+    int kin() const { return pad8(n_in); }
+    int kh() const { return pad8(H); }
+    int kout() const { return pad8(n_out); }
 
-    // refresh the transposed bf16 weights from the fp32 masters
-    void transpose_weights(hipStream_t st)
+    // the bf16 copies from the fp32 masters, after an Adam step (a) or without
+    void refresh_weights(hipStream_t st, const AdamArgs* a)
     {
-        if (!kc) return;
-        auto tr = [&](size_t off, int K, int N) {
-            const dim3 grid((N + 31) / 32, (K + 31) / 32);
-            k_transpose_bf16<<<grid, 256, 0, st>>>(w + off, K, N, wt + off);
+        auto layer = [&](size_t off, int K, int N, __bf16* Wt, long long ldt, __bf16* Wn, long long ldn) {
+            const dim3 grid((N + 63) / 64, (K + 63) / 64);
+            k_weights<<<grid, 256, 0, st>>>(w + off, a ? m + off : nullptr, v + off, g + off, K, N, a ? *a : AdamArgs{},
+                                            Wt, ldt, Wn, ldn);
         };
-        tr(o_W1, n_in, H);
-        tr(o_W2, H, H);
-        tr(o_W3, H, n_out);
+        layer(o_W1, n_in, H, W1t, kin(), nullptr, 0);
+        layer(o_W2, H, H, W2t, kh(), W2n, kh());
+        layer(o_W3, H, n_out, W3t, kh(), W3n, kout());
+        if (a) {
+            const BiasSegs b{{static_cast<long long>(o_b1), static_cast<long long>(o_b2), static_cast<long long>(o_b3)},
+                             {H, H, n_out}};
+            k_adam_bias<<<blocks_for(2LL * H + n_out, 256), 256, 0, st>>>(w, m, v, g, b, *a);
+        }
         HIPCHK(hipGetLastError());
     }
 
@@ -86,40 +88,96 @@ struct g2g_mlp_s {
         if (M <= ws_M) return;
         HIPCHK(hipStreamSynchronize(stream));
         ws.release();
-        const size_t m = static_cast<size_t>(M);
-        X = ws.get<__bf16>(m * n_in);
-        Z1 = ws.get<float>(m * H);
-        Z2 = ws.get<float>(m * H);
-        H1 = ws.get<__bf16>(m * H);
-        H2 = ws.get<__bf16>(m * H);
-        Y = ws.get<float>(m * n_out);
-        T = ws.get<float>(m * n_out);
-        dY = ws.get<float>(m * n_out);
-        dYb = ws.get<__bf16>(m * n_out);
-        dZ1 = ws.get<float>(m * H);
-        dZ2 = ws.get<float>(m * H);
-        dZ1b = ws.get<__bf16>(m * H);
-        dZ2b = ws.get<__bf16>(m * H);
-        loss = ws.get<float>(1);
+        ws_M = 0;
+        const size_t r = static_cast<size_t>(M);
+        // (padding columns are zeroed once and never written)
+        auto padded = [&](size_t cols, size_t pitch) {
+            __bf16* p = ws.get<__bf16>(r * pitch);
+            if (cols != pitch) HIPCHK(hipMemsetAsync(p, 0, r * pitch * sizeof(__bf16), stream));
+            return p;
+        };
+        X = padded(n_in, kin());
+        H1 = padded(H, kh());
+        H2 = padded(H, kh());
+        Y = ws.get<float>(r * n_out);
         ws_M = M;
+    }
+
+    // waves of a product's launch, at most: 64 x 64 outputs each or (split)
+    // 32 x 32, in workgroups of 128 x 128
+    static size_t waves(int M, int N)
+    {
+        return 16 * static_cast<size_t>((M + 127) / 128) * static_cast<size_t>((N + 127) / 128);
+    }
+
+    void train_workspace(int M)
+    {
+        workspace(M);
+        if (M <= tr_M) return;
+        HIPCHK(hipStreamSynchronize(stream));
+        tr.release();
+        tr_M = 0;
+        const size_t r = static_cast<size_t>(M), mt = static_cast<size_t>(pad8(M)), rb = (r + 31) / 32;
+        Z1 = tr.get<float>(r * H);
+        Z2 = tr.get<float>(r * H);
+        T = tr.get<float>(r * n_out);
+        Xt = tr.get<__bf16>(mt * n_in);
+        H1t = tr.get<__bf16>(mt * H);
+        H2t = tr.get<__bf16>(mt * H);
+        dYb = tr.get<__bf16>(r * kout());
+        dYt = tr.get<__bf16>(mt * n_out);
+        dZ2b = tr.get<__bf16>(r * kh());
+        dZ2t = tr.get<__bf16>(mt * H);
+        dZ1t = tr.get<__bf16>(mt * H);
+        HIPCHK(hipMemsetAsync(dYb, 0, r * kout() * sizeof(__bf16), stream));
+        HIPCHK(hipMemsetAsync(dZ2b, 0, r * kh() * sizeof(__bf16), stream));
+        cs1 = tr.get<float>(rb * H);
+        cs2 = tr.get<float>(rb * H);
+        cs3 = tr.get<float>(rb * n_out);
+        sums = tr.get<float>(waves(n_in, H) + waves(H, H) + waves(H, n_out) +
+                             blocks_for(2LL * H + n_out, 256));
+        loss_sums = tr.get<float>(waves(M, n_out));
+        if (!loss) loss = own.get<float>(2);
+        tr_M = M;
+    }
+
+    float* partials(size_t n)
+    {
+        if (n > part_cap) {
+            HIPCHK(hipStreamSynchronize(stream));
+            pt.release();
+            part_cap = 0;
+            part = pt.get<float>(n);
+            part_cap = n;
+        }
+        return part;
     }
 };
 
 namespace {
 
-template <bool TA, bool TB, int EPI>
+template <bool TA, bool TB>
 void gemm(hipStream_t st, const __bf16* A, long long lda, const __bf16* B, long long ldb, int M, int N, int K,
-          float* C, long long ldc, __bf16* Hh = nullptr, long long ldh = 0, float* Z = nullptr, long long ldz = 0,
-          const float* bias = nullptr)
+          float* C, long long ldc)
 {
-    GemmArgs a{A, lda, B, ldb, M, N, K, C, ldc, Hh, ldh, Z, ldz, bias};
+    GemmArgs a{};
+    a.A = A;
+    a.lda = lda;
+    a.B = B;
+    a.ldb = ldb;
+    a.M = M;
+    a.N = N;
+    a.K = K;
+    a.C = C;
+    a.ldc = ldc;
     const dim3 grid((N + 127) / 128, (M + 127) / 128);
-    k_gemm<TA, TB, EPI><<<grid, 256, 0, st>>>(a);
+    k_gemm<TA, TB><<<grid, 256, 0, st>>>(a);
     HIPCHK(hipGetLastError());
 }
 
-// X (fp32, M x n_in, host or device) -> the workspace's bf16 X
-void stage_x(g2g_mlp_s* p, const float* X, int M, int on_device)
+// X (fp32, M x n_in, host or device) -> the workspace's bf16 X and, for a
+// training step, its transpose
+void stage_x(g2g_mlp_s* p, const float* X, int M, int on_device, bool train)
 {
     const size_t n = static_cast<size_t>(M) * p->n_in;
     const float* src = X;
@@ -129,85 +187,151 @@ void stage_x(g2g_mlp_s* p, const float* X, int M, int on_device)
         HIPCHK(hipMemcpyAsync(d, X, n * sizeof(float), hipMemcpyHostToDevice, p->stream));
         src = d;
     }
-    k_f32_to_bf16<<<blocks_for(static_cast<long long>(n), 256), 256, 0, p->stream>>>(src, static_cast<long long>(n),
-                                                                                     p->X);
+    const dim3 grid((p->n_in + 63) / 64, (M + 63) / 64);
+    k_stage_x<<<grid, 256, 0, p->stream>>>(src, M, p->n_in, p->X, p->kin(), train ? p->Xt : nullptr,
+                                           g2g_mlp_s::pad8(M));
     HIPCHK(hipGetLastError());
     if (!on_device) HIPCHK(hipStreamSynchronize(p->stream));
 }
 
+// C = A B^T (A M x K, B N x K).  Fewer than half a tile per CU: K is split so
+// that the launch covers the CUs (at least 256 of K a split), the partials
+// summed, in order, by a second launch that runs the epilogue.  Returns the
+// floats written to `sums`.
 template <int EPI>
-void gemm_kc(hipStream_t st, const __bf16* A, long long lda, const __bf16* Bt, long long ldb, int M, int N, int K,
-             float* C, long long ldc, __bf16* Hh, long long ldh, float* Z, long long ldz, const float* bias)
+size_t product(g2g_mlp_s* p, GemmArgs a)
 {
-    GemmArgs a{A, lda, Bt, ldb, M, N, K, C, ldc, Hh, ldh, Z, ldz, bias};
-    const dim3 grid((N + 127) / 128, (M + 127) / 128);
-    k_gemm_kc<EPI><<<grid, 256, 0, st>>>(a);
-    HIPCHK(hipGetLastError());
-}
-
-// forward of the staged X into p->Y; keep_z: the pre-activations the backward
-// pass needs (inference skips them)
-void forward(g2g_mlp_s* p, int M, bool keep_z = true)
-{
-    if (p->kc) {
-        gemm_kc<kEpiBiasGeluBf16>(p->stream, p->X, p->n_in, p->W1t(), p->n_in, M, p->H, p->n_in, nullptr, 0, p->H1,
-                                  p->H, keep_z ? p->Z1 : nullptr, p->H, p->w + p->o_b1);
-        gemm_kc<kEpiBiasGeluBf16>(p->stream, p->H1, p->H, p->W2t(), p->H, M, p->H, p->H, nullptr, 0, p->H2, p->H,
-                                  keep_z ? p->Z2 : nullptr, p->H, p->w + p->o_b2);
-        gemm_kc<kEpiBiasF32>(p->stream, p->H2, p->H, p->W3t(), p->H, M, p->n_out, p->H, p->Y, p->n_out, nullptr, 0,
-                             nullptr, 0, p->w + p->o_b3);
-        return;
+    constexpr int kCus = 256, kMinK = 256;
+    const int gx = (a.N + 127) / 128, gy = (a.M + 127) / 128, tiles = gx * gy;
+    int splits = tiles >= kCus / 2 ? 1 : std::min(kCus / tiles, a.K / kMinK);
+    if (splits <= 1) {
+        k_gemm_kc<EPI><<<dim3(gx, gy), 256, 0, p->stream>>>(a);
+        HIPCHK(hipGetLastError());
+        return 4 * static_cast<size_t>(tiles);
     }
-    gemm<false, false, kEpiBiasGeluBf16>(p->stream, p->X, p->n_in, p->W1b(), p->H, M, p->H, p->n_in, nullptr, 0,
-                                         p->H1, p->H, p->Z1, p->H, p->w + p->o_b1);
-    gemm<false, false, kEpiBiasGeluBf16>(p->stream, p->H1, p->H, p->W2b(), p->H, M, p->H, p->H, nullptr, 0, p->H2,
-                                         p->H, p->Z2, p->H, p->w + p->o_b2);
-    gemm<false, false, kEpiBiasF32>(p->stream, p->H2, p->H, p->W3b(), p->n_out, M, p->n_out, p->H, p->Y, p->n_out,
-                                    nullptr, 0, nullptr, 0, p->w + p->o_b3);
+    GemmArgs s = a;
+    s.k_split = (((a.K + splits - 1) / splits) + 63) / 64 * 64;
+    splits = (a.K + s.k_split - 1) / s.k_split;
+    s.C = p->partials(static_cast<size_t>(splits) * a.M * a.N);
+    s.ldc = a.N;
+    k_gemm_kc<kEpiF32><<<dim3(gx, gy, splits), 256, 0, p->stream>>>(s);
+    const dim3 grid((a.N + 31) / 32, (a.M + 31) / 32);
+    k_gemm_sum<EPI><<<grid, 64, 0, p->stream>>>(a, s.C, splits);
+    HIPCHK(hipGetLastError());
+    return static_cast<size_t>(grid.x) * grid.y;
 }
 
-// out[n] = sum over the M rows of X[m][n]
-void colsum(hipStream_t st, const float* X, long long ldx, int M, int N, float* out)
+GemmArgs operands(const __bf16* A, long long lda, const __bf16* B, long long ldb, int M, int N, int K)
 {
-    HIPCHK(hipMemsetAsync(out, 0, static_cast<size_t>(N) * sizeof(float), st));
-    const dim3 grid((N + 63) / 64, (M + kColRows - 1) / kColRows);
-    k_colsum<<<grid, 256, 0, st>>>(X, ldx, M, N, out);
+    GemmArgs a{};
+    a.A = A;
+    a.lda = lda;
+    a.B = B;
+    a.ldb = ldb;
+    a.M = M;
+    a.N = N;
+    a.K = K;
+    return a;
+}
+
+// the hidden layers of the staged X; train: with the pre-activations and
+// transposes the backward pass needs
+void hidden(g2g_mlp_s* p, int M, bool train)
+{
+    const int mt = g2g_mlp_s::pad8(M);
+    auto layer = [&](const __bf16* A, int ka, const __bf16* Wt, size_t o_b, __bf16* Hh, __bf16* Ht, float* Z) {
+        GemmArgs a = operands(A, ka, Wt, ka, M, p->H, ka);
+        a.bias = p->w + o_b;
+        a.H = Hh;
+        a.ldh = p->kh();
+        a.Ht = train ? Ht : nullptr;
+        a.Mt = mt;
+        a.Z = train ? Z : nullptr;
+        a.ldz = p->H;
+        product<kEpiGelu>(p, a);
+    };
+    layer(p->X, p->kin(), p->W1t, p->o_b1, p->H1, p->H1t, p->Z1);
+    layer(p->H1, p->kh(), p->W2t, p->o_b2, p->H2, p->H2t, p->Z2);
+}
+
+// inference of the staged X into Y
+void forward(g2g_mlp_s* p, int M, float* Y)
+{
+    hidden(p, M, false);
+    GemmArgs a = operands(p->H2, p->kh(), p->W3t, p->kh(), M, p->n_out, p->kh());
+    a.bias = p->w + p->o_b3;
+    a.C = Y;
+    a.ldc = p->n_out;
+    product<kEpiBiasF32>(p, a);
+}
+
+// loss (p->loss[0]) and gradients (p->g), with their squared norm
+// (p->loss[1]), of the staged X against the targets T (device)
+void loss_and_grads(g2g_mlp_s* p, const float* T, int M)
+{
+    const int mt = g2g_mlp_s::pad8(M), H = p->H;
+    hidden(p, M, true);
+    // output layer: the loss's derivative straight from the product
+    const float scale = static_cast<float>(1.0 / (static_cast<double>(M) * p->n_out));
+    GemmArgs a = operands(p->H2, p->kh(), p->W3t, p->kh(), M, p->n_out, p->kh());
+    a.bias = p->w + p->o_b3;
+    a.T = T;
+    a.ldc = p->n_out;
+    a.scale = scale;
+    a.H = p->dYb;
+    a.ldh = p->kout();
+    a.Ht = p->dYt;
+    a.Mt = mt;
+    a.colsum = p->cs3;
+    a.sums = p->loss_sums;
+    const size_t n_loss = product<kEpiMse>(p, a);
+    size_t n_sums = 0;
+    auto grad = [&](const __bf16* A, int rows, const __bf16* B, int cols, size_t off) {
+        GemmArgs q = operands(A, mt, B, mt, rows, cols, mt);
+        q.C = p->g + off;
+        q.ldc = cols;
+        q.sums = p->sums + n_sums;
+        n_sums += product<kEpiGrad>(p, q);
+    };
+    auto back = [&](const __bf16* A, int ka, const __bf16* Wn, __bf16* Hh, __bf16* Ht, float* Z, float* cs) {
+        GemmArgs q = operands(A, ka, Wn, ka, M, H, ka);
+        q.H = Hh;
+        q.ldh = p->kh();
+        q.Ht = Ht;
+        q.Mt = mt;
+        q.Z = Z;
+        q.ldz = H;
+        q.colsum = cs;
+        product<kEpiGeluBwd>(p, q);
+    };
+    grad(p->H2t, H, p->dYt, p->n_out, p->o_W3);
+    back(p->dYb, p->kout(), p->W3n, p->dZ2b, p->dZ2t, p->Z2, p->cs2);
+    grad(p->H1t, H, p->dZ2t, H, p->o_W2);
+    back(p->dZ2b, p->kh(), p->W2n, nullptr, p->dZ1t, p->Z1, p->cs1);
+    grad(p->Xt, p->n_in, p->dZ1t, H, p->o_W1);
+    const BiasGradArgs b{{{static_cast<long long>(p->o_b1), static_cast<long long>(p->o_b2),
+                           static_cast<long long>(p->o_b3)},
+                          {H, H, p->n_out}},
+                         {p->cs1, p->cs2, p->cs3},
+                         (M + 31) / 32,
+                         p->g,
+                         p->sums + n_sums};
+    const unsigned nb = blocks_for(2LL * H + p->n_out, 256);
+    k_bias_grad<<<nb, 256, 0, p->stream>>>(b);
+    n_sums += nb;
+    k_finish<<<1, 1024, 0, p->stream>>>(p->loss_sums, static_cast<int>(n_loss), scale, p->sums,
+                                        static_cast<int>(n_sums), p->loss, p->loss + 1);
     HIPCHK(hipGetLastError());
 }
 
-// loss and gradients (into p->g) of the staged X against targets p->T
-void backward(g2g_mlp_s* p, int M)
+// the targets on the device: the caller's array, or its staged host copy
+const float* stage_t(g2g_mlp_s* p, const float* T, int M, int on_device)
 {
-    hipStream_t st = p->stream;
-    const long long ne = static_cast<long long>(M) * p->n_out;
-    HIPCHK(hipMemsetAsync(p->loss, 0, sizeof(float), st));
-    k_mse_grad<<<std::min<unsigned>(blocks_for(ne, 256), 2048), 256, 0, st>>>(p->Y, p->T, ne,
-                                                                              1.0f / static_cast<float>(ne), p->dY,
-                                                                              p->dYb,
-                                                    p->loss);
-    HIPCHK(hipGetLastError());
-    // layer 3: dW3 = H2^T dY, db3 = sum dY, dZ2 = (dY W3^T) gelu'(Z2)
-    gemm<true, false, kEpiF32>(st, p->H2, p->H, p->dYb, p->n_out, p->H, p->n_out, M, p->g + p->o_W3, p->n_out);
-    colsum(st, p->dY, p->n_out, M, p->n_out, p->g + p->o_b3);
-    gemm<false, true, kEpiGeluBwd>(st, p->dYb, p->n_out, p->W3b(), p->n_out, M, p->H, p->n_out, p->dZ2, p->H,
-                                   p->dZ2b, p->H, p->Z2, p->H);
-    // layer 2
-    gemm<true, false, kEpiF32>(st, p->H1, p->H, p->dZ2b, p->H, p->H, p->H, M, p->g + p->o_W2, p->H);
-    colsum(st, p->dZ2, p->H, M, p->H, p->g + p->o_b2);
-    gemm<false, true, kEpiGeluBwd>(st, p->dZ2b, p->H, p->W2b(), p->H, M, p->H, p->H, p->dZ1, p->H, p->dZ1b, p->H,
-                                   p->Z1, p->H);
-    // layer 1
-    gemm<true, false, kEpiF32>(st, p->X, p->n_in, p->dZ1b, p->H, p->n_in, p->H, M, p->g + p->o_W1, p->H);
-    colsum(st, p->dZ1, p->H, M, p->H, p->g + p->o_b1);
-    HIPCHK(hipGetLastError());
-}
-
-void stage_t(g2g_mlp_s* p, const float* T, int M, int on_device)
-{
+    if (on_device) return T;
     const size_t n = static_cast<size_t>(M) * p->n_out;
-    HIPCHK(hipMemcpyAsync(p->T, T, n * sizeof(float), on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice,
-                          p->stream));
-    if (!on_device) HIPCHK(hipStreamSynchronize(p->stream));
+    HIPCHK(hipMemcpyAsync(p->T, T, n * sizeof(float), hipMemcpyHostToDevice, p->stream));
+    HIPCHK(hipStreamSynchronize(p->stream));
+    return p->T;
 }
 
 }  // namespace
@@ -227,12 +351,12 @@ void mlp_warm_start_tiles(g2g_mlp_s* p, const double2* S_tiles, int M, int n, co
     p->stream = st;
     p->workspace(M);
     const dim3 patches((n + kPatchBuses - 1) / kPatchBuses, (M + 63) / 64);
-    k_features_tiles_t<<<patches, 256, 0, st>>>(S_tiles, M, n, p->in_mu, p->in_sigma, p->X, p->n_in);
+    k_features_tiles_t<<<patches, 256, 0, st>>>(S_tiles, M, n, p->in_mu, p->in_sigma, p->X, p->kin());
     if (n_mask > 0)
         k_mask_features<<<blocks_for(static_cast<long long>(M) * n_mask, 256), 256, 0, st>>>(d_mask, M, n, n_mask,
-                                                                                            p->X, p->n_in);
+                                                                                            p->X, p->kin());
     HIPCHK(hipGetLastError());
-    forward(p, M, false);
+    forward(p, M, p->Y);
     k_warm_v_tiles_t<<<patches, 256, 0, st>>>(p->Y, p->n_out, M, n, p->out_mu, p->out_sigma, p->vfix, p->kind,
                                               V_tiles);
     HIPCHK(hipGetLastError());
@@ -266,9 +390,11 @@ int g2g_mlp_create(int32_t n_in, int32_t n_hidden, int32_t n_out, uint64_t seed,
         p->m = p->own.get<float>(o);
         p->v = p->own.get<float>(o);
         p->g = p->own.get<float>(o);
-        p->wb = p->own.get<__bf16>(o);
-        p->kc = n_in % 8 == 0 && n_hidden % 8 == 0 && n_out % 8 == 0;
-        if (p->kc) p->wt = p->own.get<__bf16>(o);
+        p->W1t = p->own.get<__bf16>(static_cast<size_t>(n_hidden) * p->kin());
+        p->W2t = p->own.get<__bf16>(static_cast<size_t>(n_hidden) * p->kh());
+        p->W3t = p->own.get<__bf16>(static_cast<size_t>(n_out) * p->kh());
+        p->W2n = p->own.get<__bf16>(static_cast<size_t>(n_hidden) * p->kh());
+        p->W3n = p->own.get<__bf16>(static_cast<size_t>(n_hidden) * p->kout());
         // Glorot-uniform weights, zero biases (seeded)
         std::vector<float> h(o, 0.0f);
         std::mt19937_64 rng(seed);
@@ -286,9 +412,7 @@ int g2g_mlp_create(int32_t n_in, int32_t n_hidden, int32_t n_out, uint64_t seed,
         // the layers' gradients never write the padding between them, which
         // the gradient norm and the Adam update read: zero it once
         HIPCHK(hipMemset(p->g, 0, o * sizeof(float)));
-        k_f32_to_bf16<<<blocks_for(static_cast<long long>(o), 256), 256>>>(p->w, static_cast<long long>(o), p->wb);
-        HIPCHK(hipGetLastError());
-        p->transpose_weights(nullptr);
+        p->refresh_weights(nullptr, nullptr);
         HIPCHK(hipDeviceSynchronize());
         *out = p.release();
     });
@@ -335,9 +459,7 @@ int g2g_mlp_set_params(g2g_mlp_t p, const float* in, int64_t n)
         if (n != static_cast<int64_t>(p->n_params)) throw std::invalid_argument("parameter count mismatch");
         HIPCHK(hipStreamSynchronize(p->stream));
         HIPCHK(hipMemcpy(p->w, in, p->n_params * sizeof(float), hipMemcpyHostToDevice));
-        k_f32_to_bf16<<<blocks_for(static_cast<long long>(n), 256), 256, 0, p->stream>>>(p->w, n, p->wb);
-        HIPCHK(hipGetLastError());
-        p->transpose_weights(p->stream);
+        p->refresh_weights(p->stream, nullptr);
         HIPCHK(hipStreamSynchronize(p->stream));
     });
 }
@@ -377,10 +499,11 @@ int g2g_mlp_forward(g2g_mlp_t p, const float* X, int32_t M, float* Y, int32_t on
         if (!p || !X || !Y) throw std::invalid_argument("null argument");
         if (M <= 0) throw std::invalid_argument("M must be positive");
         p->workspace(M);
-        stage_x(p, X, M, on_device);
-        forward(p, M, false);
-        HIPCHK(hipMemcpyAsync(Y, p->Y, static_cast<size_t>(M) * p->n_out * sizeof(float),
-                              on_device ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, p->stream));
+        stage_x(p, X, M, on_device, false);
+        forward(p, M, on_device ? Y : p->Y);
+        if (!on_device)
+            HIPCHK(hipMemcpyAsync(Y, p->Y, static_cast<size_t>(M) * p->n_out * sizeof(float), hipMemcpyDeviceToHost,
+                                  p->stream));
         HIPCHK(hipStreamSynchronize(p->stream));
     });
 }
@@ -391,11 +514,9 @@ int g2g_mlp_loss_grad(g2g_mlp_t p, const float* X, const float* T, int32_t M, fl
     return guarded([&] {
         if (!p || !X || !T) throw std::invalid_argument("null argument");
         if (M <= 0) throw std::invalid_argument("M must be positive");
-        p->workspace(M);
-        stage_x(p, X, M, on_device);
-        stage_t(p, T, M, on_device);
-        forward(p, M);
-        backward(p, M);
+        p->train_workspace(M);
+        stage_x(p, X, M, on_device, true);
+        loss_and_grads(p, stage_t(p, T, M, on_device), M);
         if (loss) HIPCHK(hipMemcpyAsync(loss, p->loss, sizeof(float), hipMemcpyDeviceToHost, p->stream));
         if (grads)
             HIPCHK(hipMemcpyAsync(grads, p->g, p->n_params * sizeof(float), hipMemcpyDeviceToHost, p->stream));
@@ -409,25 +530,15 @@ int g2g_mlp_train_step(g2g_mlp_t p, const float* X, const float* T, int32_t M, f
     return guarded([&] {
         if (!p || !X || !T) throw std::invalid_argument("null argument");
         if (M <= 0) throw std::invalid_argument("M must be positive");
-        p->workspace(M);
-        stage_x(p, X, M, on_device);
-        stage_t(p, T, M, on_device);
-        forward(p, M);
-        backward(p, M);
+        p->train_workspace(M);
+        stage_x(p, X, M, on_device, true);
+        loss_and_grads(p, stage_t(p, T, M, on_device), M);
         ++p->step;
         const float b1 = 0.9f, b2 = 0.999f;
         const float c1 = 1.0f / (1.0f - std::pow(b1, static_cast<float>(p->step)));
         const float c2 = 1.0f / (1.0f - std::pow(b2, static_cast<float>(p->step)));
-        const long long n = static_cast<long long>(p->n_params);
-        if (p->clip > 0.0f) {
-            if (!p->gnorm2) p->gnorm2 = p->own.get<float>(1);
-            k_fill_int<<<1, 64, 0, p->stream>>>(reinterpret_cast<int*>(p->gnorm2), 0, 1);  // 0.0f
-            k_sumsq<<<std::min<long long>(1024, blocks_for(n, 256)), 256, 0, p->stream>>>(p->g, n, p->gnorm2);
-        }
-        k_adam<<<blocks_for(n, 256), 256, 0, p->stream>>>(p->w, p->m, p->v, p->g, n, lr, b1, b2, 1e-8f, c1, c2, p->wb,
-                                                           p->clip > 0.0f ? p->gnorm2 : nullptr, p->clip);
-        HIPCHK(hipGetLastError());
-        p->transpose_weights(p->stream);
+        const AdamArgs a{lr, b1, b2, 1e-8f, c1, c2, p->clip > 0.0f ? p->loss + 1 : nullptr, p->clip};
+        p->refresh_weights(p->stream, &a);
         if (loss) {
             HIPCHK(hipMemcpyAsync(loss, p->loss, sizeof(float), hipMemcpyDeviceToHost, p->stream));
             HIPCHK(hipStreamSynchronize(p->stream));
@@ -458,12 +569,18 @@ int g2g_gemm_bf16(int32_t trans_a, int32_t trans_b, int32_t M, int32_t N, int32_
         float* dC = s.get<float>(static_cast<size_t>(M) * ldc);
         HIPCHK(hipMemcpy(dA, A, na * 2, hipMemcpyHostToDevice));
         HIPCHK(hipMemcpy(dB, B, nb * 2, hipMemcpyHostToDevice));
-        if (!trans_a && !trans_b) gemm<false, false, kEpiF32>(nullptr, dA, lda, dB, ldb, M, N, K, dC, ldc);
+        if (!trans_a && !trans_b) gemm<false, false>(nullptr, dA, lda, dB, ldb, M, N, K, dC, ldc);
         else if (!trans_a && trans_b && K % 8 == 0 && lda % 8 == 0 && ldb % 8 == 0)
-            gemm_kc<kEpiF32>(nullptr, dA, lda, dB, ldb, M, N, K, dC, ldc, nullptr, 0, nullptr, 0, nullptr);
-        else if (!trans_a && trans_b) gemm<false, true, kEpiF32>(nullptr, dA, lda, dB, ldb, M, N, K, dC, ldc);
-        else if (trans_a && !trans_b) gemm<true, false, kEpiF32>(nullptr, dA, lda, dB, ldb, M, N, K, dC, ldc);
-        else gemm<true, true, kEpiF32>(nullptr, dA, lda, dB, ldb, M, N, K, dC, ldc);
+        {
+            GemmArgs a = operands(dA, lda, dB, ldb, M, N, K);
+            a.C = dC;
+            a.ldc = ldc;
+            k_gemm_kc<kEpiF32><<<dim3((N + 127) / 128, (M + 127) / 128), 256>>>(a);
+            HIPCHK(hipGetLastError());
+        }
+        else if (!trans_a && trans_b) gemm<false, true>(nullptr, dA, lda, dB, ldb, M, N, K, dC, ldc);
+        else if (trans_a && !trans_b) gemm<true, false>(nullptr, dA, lda, dB, ldb, M, N, K, dC, ldc);
+        else gemm<true, true>(nullptr, dA, lda, dB, ldb, M, N, K, dC, ldc);
         HIPCHK(hipDeviceSynchronize());
         HIPCHK(hipMemcpy(C, dC, static_cast<size_t>(M) * ldc * sizeof(float), hipMemcpyDeviceToHost));
     });
