@@ -1249,12 +1249,16 @@ public:
         need_run();
         if (!br_.set) throw std::runtime_error("call set_branch_data() first");
         const int n = n_bus(), m = br_.m(), rows = n_rows();
-        or_.assign(static_cast<size_t>(rows) * m, std::nan(""));
-        ex_.assign(static_cast<size_t>(rows) * m, std::nan(""));
         const std::vector<cplx> y4 = br_.y4();
         std::vector<int> live;
         for (int r = 0; r < rows; ++r)
             if (res_.status[r] != static_cast<int32_t>(RowStatus::NotSimulated)) live.push_back(r);
+        // rows x m on the device, where they stay until they are asked for
+        const size_t bytes = static_cast<size_t>(rows) * m * sizeof(double);
+        ensure(dOr_, bytes);
+        ensure(dEx_, bytes);
+        flow_rows_ = rows;
+        flow_m_ = m;
         if (live.empty()) return;
         const int cap = std::min<int>(std::max(1, batch_size_), static_cast<int>(live.size()));
         if (!batch_ || batch_->rows < cap) {
@@ -1262,7 +1266,7 @@ public:
             batch_ = std::make_unique<Batch>(*grid_, cap, precision_, 0);
         }
         const int B = batch_->rows;
-        std::vector<double> o(static_cast<size_t>(B) * m), e(static_cast<size_t>(B) * m);
+        DevBufPtr o, e;  // a chunk's rows, when they are not consecutive
         std::vector<int32_t> tp, tb;
         for (size_t c0 = 0; c0 < live.size(); c0 += B) {
             const int k = static_cast<int>(std::min<size_t>(B, live.size() - c0));
@@ -1275,23 +1279,32 @@ public:
                 tp.push_back(static_cast<int32_t>(tb.size()));
             }
             check(g2g_batch_set_active_rows(batch_->h, k));
-            for (const auto& rn : row_runs(live, c0, k))  // the rows' results, device to device
+            const auto runs = row_runs(live, c0, k);
+            for (const auto& rn : runs)  // the rows' results, device to device
                 check(g2g_batch_set_v(batch_->h, reinterpret_cast<const double*>(dVres_->c() + static_cast<size_t>(rn[0]) * n),
                                       n, rn[1], rn[2], 1));
+            const size_t row = static_cast<size_t>(m) * sizeof(double);
+            auto at = [&](const DevBufPtr& b, size_t r) { return static_cast<unsigned char*>(b->p) + r * row; };
+            const bool straight = runs.size() == 1;
+            if (!straight) {
+                ensure(o, static_cast<size_t>(B) * row);
+                ensure(e, static_cast<size_t>(B) * row);
+            }
             check(g2g_batch_branch_flows(batch_->h, m, br_.f.data(), br_.t.data(),
                                          reinterpret_cast<const double*>(y4.data()), br_.base_or.data(),
-                                         br_.base_ex.data(), tp.data(), tb.empty() ? nullptr : tb.data(), o.data(),
-                                         e.data()));
-            for (int q = 0; q < k; ++q) {
-                const int r = live[c0 + q];
-                std::copy_n(o.begin() + static_cast<size_t>(q) * m, m, or_.begin() + static_cast<size_t>(r) * m);
-                std::copy_n(e.begin() + static_cast<size_t>(q) * m, m, ex_.begin() + static_cast<size_t>(r) * m);
+                                         br_.base_ex.data(), tp.data(), tb.empty() ? nullptr : tb.data(),
+                                         reinterpret_cast<double*>(straight ? at(dOr_, runs[0][0]) : at(o, 0)),
+                                         reinterpret_cast<double*>(straight ? at(dEx_, runs[0][0]) : at(e, 0))));
+            for (const auto& rn : runs) {
+                if (straight) break;
+                hipchk(hipMemcpy(at(dOr_, rn[0]), at(o, rn[2]), rn[1] * row, hipMemcpyDeviceToDevice), "hipMemcpy D2D");
+                hipchk(hipMemcpy(at(dEx_, rn[0]), at(e, rn[2]), rn[1] * row, hipMemcpyDeviceToDevice), "hipMemcpy D2D");
             }
         }
         flows_ = true;
     }
-    py::array_t<double> get_or_amps() const { return flows(or_); }
-    py::array_t<double> get_ex_amps() const { return flows(ex_); }
+    py::array_t<double> get_or_amps() const { return flows(dOr_); }
+    py::array_t<double> get_ex_amps() const { return flows(dEx_); }
 
     CArr v_base() const
     {
@@ -1307,16 +1320,25 @@ protected:
     {
         if (!ran_) throw std::runtime_error("call run() first");
     }
-    py::array_t<double> flows(const std::vector<double>& v) const
+    // a host copy of a flow result; rows not simulated read NaN
+    py::array_t<double> flows(const DevBufPtr& d) const
     {
         if (!flows_) throw std::runtime_error("call compute_flows() first");
-        py::array_t<double> a({static_cast<py::ssize_t>(n_rows()), static_cast<py::ssize_t>(br_.m())});
-        std::copy(v.begin(), v.end(), a.mutable_data());
+        const size_t m = static_cast<size_t>(flow_m_);
+        py::array_t<double> a({static_cast<py::ssize_t>(flow_rows_), static_cast<py::ssize_t>(m)});
+        double* p = a.mutable_data();
+        if (flow_rows_ > 0 && m > 0)
+            hipchk(hipMemcpy(p, d->p, static_cast<size_t>(flow_rows_) * m * sizeof(double), hipMemcpyDeviceToHost),
+                   "hipMemcpy D2H");
+        for (int r = 0; r < flow_rows_; ++r)
+            if (res_.status[r] == static_cast<int32_t>(RowStatus::NotSimulated))
+                std::fill_n(p + static_cast<size_t>(r) * m, m, std::nan(""));
         return a;
     }
     Branches br_;
     std::vector<std::vector<int>> trips_;  // tripped branches per row
-    std::vector<double> or_, ex_;
+    DevBufPtr dOr_, dEx_;                  // branch currents, rows x m
+    int flow_rows_ = 0, flow_m_ = 0;
     bool flows_ = false;
 
     std::unique_ptr<Grid> grid_;

@@ -77,8 +77,11 @@ __global__ void k_fill_int(int* p, int v, long long n);
 __global__ void k_add_int(int* p, int v);
 __global__ void k_count_tiles(const int* status, int rows_pad, int* tile_active);
 __global__ void k_branch_flows(const double2* V, int n, const int* from, const int* to, const double2* y4,
-                               const double* base_or, const double* base_ex, int m, int T, double* or_t,
-                               double* ex_t);
+                               const double* base_or, const double* base_ex, int m, int rows, double* or_amps,
+                               double* ex_amps);
+__global__ void k_trip_flows(const int* trip_ptr, const int* trip, int rows, int m, double* or_amps,
+                             double* ex_amps);
+__global__ void k_init_rows(int active, int rows_pad, int* status, int* iters, int* tile_active);
 __global__ void k_limit_violations(ViolationArgs a);
 size_t limit_violations_lds(int K);
 template <typename T>
@@ -338,6 +341,8 @@ struct g2g_plan_s {
     }
 };
 
+constexpr size_t kPinnedUpload = 128 << 10;  // bytes of a pinned upload half
+
 // staging buffers of the streamed-row calls
 enum StageBuf { kStSlots, kStS, kStV, kStEdPtr, kStEdEnt, kStEdDelta, kStMask, kStSg, kStVg, kStageBufs };
 
@@ -376,7 +381,16 @@ struct g2g_batch_s {
     int* n_active = nullptr;  // rows and tiles still iterating (2 ints)
     int* clamped = nullptr;
     int* error = nullptr;     // stream kernels' give-up flag
-    int* h_active = nullptr;  // pinned: rows and tiles still iterating, rows restarted; [4..8]: row_cnt
+    // one pinned allocation: h_active {rows and tiles still iterating, rows
+    // restarted; [4..8] row_cnt; [9] error}, the staging halves of small Sbus /
+    // V uploads, and the results (status, iterations, residuals) of rows_pad rows
+    int* h_active = nullptr;
+    unsigned char* h_up[2] = {nullptr, nullptr};
+    bool up_pending[2] = {false, false};  // a staged upload may still be read
+    int* h_status = nullptr;
+    int* h_iters = nullptr;
+    double* h_res = nullptr;
+    bool solve_read = false;  // the solve's error flag and statuses are in h_active / h_status
     // warm solves: the caller's start voltages (the fallback start)
     double2* V0 = nullptr;
     bool v0_row = false;  // V0 holds one row [n] (every row's fallback start is the same)
@@ -1163,14 +1177,27 @@ void launch_mismatch(g2g_batch_s* b, bool with_j, int iter, int max_iter, double
 
 void reset_rows(g2g_batch_s* b)
 {
-    // status: active for [0, active_rows), not simulated beyond
-    std::vector<int> st(static_cast<size_t>(b->rows_pad), kNotSimulated);
-    std::fill(st.begin(), st.begin() + b->active_rows, kActive);
-    HIPCHK(hipMemcpyAsync(b->status, st.data(), st.size() * sizeof(int), hipMemcpyHostToDevice, b->stream));
-    k_fill_int<<<blocks_for(b->rows_pad, 256), 256, 0, b->stream>>>(b->iters, 0, b->rows_pad);
-    k_count_tiles<<<b->T, kLanes, 0, b->stream>>>(b->status, b->rows_pad, b->tile_active);
+    k_init_rows<<<blocks_for(b->rows_pad, 256), 256, 0, b->stream>>>(b->active_rows, b->rows_pad, b->status, b->iters,
+                                                                    b->tile_active);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipStreamSynchronize(b->stream));  // st is a host temporary
+    b->solve_read = false;
+}
+
+// Waits for the stream: its staged uploads have been read.
+void sync_stream(g2g_batch_s* b)
+{
+    HIPCHK(hipStreamSynchronize(b->stream));
+    b->up_pending[0] = b->up_pending[1] = false;
+}
+
+// what a finished solve reports (the error flag, with statuses those too),
+// queued for the host behind its work
+void queue_solve_read(g2g_batch_s* b, bool statuses)
+{
+    HIPCHK(hipMemcpyAsync(b->h_active + 9, b->error, sizeof(int), hipMemcpyDeviceToHost, b->stream));
+    if (statuses && b->active_rows > 0)
+        HIPCHK(hipMemcpyAsync(b->h_status, b->status, static_cast<size_t>(b->active_rows) * sizeof(int),
+                              hipMemcpyDeviceToHost, b->stream));
 }
 
 // per-solve event bookkeeping (phase times summed over every launch)
@@ -1642,12 +1669,15 @@ int solve_rows(g2g_batch_s* b, int R, int it, bool decided, int max_iter, double
     tm.ph[1].push_back({e0, tm.mark()});
     tm.factor_main.push_back(0);
     HIPCHK(hipMemcpyAsync(b->h_active + 4, b->row_cnt, kRowCnt * sizeof(int), hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
+    const bool whole = b->compact_R == 0 && !b->mask;  // the statuses are the batch's final ones if no row is left
+    if (whole) queue_solve_read(b, true);
+    sync_stream(b);
     unsigned long long upd = 0;
     std::memcpy(&upd, b->h_active + 4, sizeof(upd));
     rows_factored += static_cast<long long>(upd);
     last_iter = std::max(last_iter, b->h_active[6]);
     const int left = b->h_active[8];
+    b->solve_read = whole && left == 0;
     if (left > 0) {
         k_count_tiles<<<b->T, kLanes, 0, st>>>(b->status, b->rows_pad, b->tile_active);
         HIPCHK(hipGetLastError());
@@ -1918,12 +1948,15 @@ void mask_islanded_v(g2g_batch_s* b)
     HIPCHK(hipGetLastError());
 }
 
-void check_stream_error(g2g_batch_s* b)
+// Waits for the work queued so far (read: that has been done, and the flag
+// read); a stream kernel that gave up is an error.
+void check_stream_error(g2g_batch_s* b, bool statuses = false, bool read = false)
 {
-    int err = 0;
-    HIPCHK(hipMemcpyAsync(&err, b->error, sizeof(int), hipMemcpyDeviceToHost, b->stream));
-    HIPCHK(hipStreamSynchronize(b->stream));
-    if (err) throw std::runtime_error("a stream wavefront gave up waiting for its data (results invalid)");
+    if (!read) {
+        queue_solve_read(b, statuses);
+        sync_stream(b);
+    }
+    if (b->h_active[9]) throw std::runtime_error("a stream wavefront gave up waiting for its data (results invalid)");
 }
 
 void fill_stats(g2g_batch_s* b, const SolveTimer& tm, int e_begin, int e_end, int iterations,
@@ -1947,9 +1980,8 @@ void fill_stats(g2g_batch_s* b, const SolveTimer& tm, int e_begin, int e_end, in
     stats->ms_factor_main = tm.ms(1, true);
     stats->rows_factored_main = tm.rows_main;
     for (char m : tm.factor_main) stats->n_factor_main += m ? 1 : 0;
-    std::vector<int> st(static_cast<size_t>(b->active_rows));
-    if (!st.empty()) HIPCHK(hipMemcpy(st.data(), b->status, st.size() * sizeof(int), hipMemcpyDeviceToHost));
-    for (int v : st) {
+    for (int r = 0; r < b->active_rows; ++r) {  // (read with the error flag)
+        const int v = b->h_status[r];
         stats->n_converged += v == kConverged;
         stats->n_maxiter += v == kMaxIter;
         stats->n_diverged += v == kDiverged;
@@ -1968,8 +2000,9 @@ void solve_impl(g2g_batch_s* b, int max_iter, double tol, int sched, g2g_solve_s
     long long rows_factored = 0;
     const int it = nr_loop<Real>(b, max_iter, tol, freeze, 0.0, tm, rows_factored);
     mask_islanded_v(b);
-    const int e_end = tm.mark();
-    check_stream_error(b);
+    // (a solve that ended in the row solver has been waited for and read)
+    const int e_end = b->solve_read ? tm.nev - 1 : tm.mark();
+    check_stream_error(b, true, b->solve_read);
     fill_stats(b, tm, e_begin, e_end, it, rows_factored, stats);
 }
 
@@ -2058,24 +2091,42 @@ void solve_warm_impl(g2g_batch_s* b, g2g_mlp_s* mlp, const unsigned char* mask, 
     b->restart_on = false;
     mask_islanded_v(b);
     const int e_end = tm.mark();
-    int R = 0;
-    HIPCHK(hipMemcpyAsync(&R, b->requeued, sizeof(int), hipMemcpyDeviceToHost, s));
-    check_stream_error(b);
+    HIPCHK(hipMemcpyAsync(b->h_active + 10, b->requeued, sizeof(int), hipMemcpyDeviceToHost, s));
+    check_stream_error(b, true);
+    const int R = b->h_active[10];
     fill_stats(b, tm, e_begin, e_end, it, rows_factored, stats);
     if (stats) stats->n_requeued = R;
 }
 
-// rows x m complex (row stride ld complex; ld = 0 broadcasts) -> tiled [T][m][64]
-void to_tiles(const double* src, long long ld, int rows, int m, int row0, int on_device, double2* dst,
-              hipStream_t st)
+template <typename T>
+T* stage_buf(g2g_batch_s* b, int i, size_t n);
+
+// Rows x m complex (row stride ld complex; ld = 0 broadcasts) -> tiled
+// [T][m][64].  Host rows of up to kPinnedUpload bytes (a power flow's or a few)
+// go through the batch's pinned half `up` and its kept device staging: no
+// allocation, and the copy need not be waited for.  Larger ones are staged in
+// memory that is given back.
+void to_tiles(g2g_batch_s* b, int up, const double* src, long long ld, int rows, int m, int row0, int on_device,
+              double2* dst)
 {
+    hipStream_t st = b->stream;
     const double2* dsrc = reinterpret_cast<const double2*>(src);
     double2* tmp = nullptr;
-    if (!on_device) {
+    if (!on_device && rows > 0) {
         const size_t cnt = ld == 0 ? static_cast<size_t>(m) : static_cast<size_t>(rows - 1) * ld + m;
-        tmp = dalloc<double2>(cnt);
-        HIPCHK(hipMemcpyAsync(tmp, src, cnt * sizeof(double2), hipMemcpyHostToDevice, st));
-        dsrc = tmp;
+        const size_t bytes = cnt * sizeof(double2);
+        if (bytes <= kPinnedUpload) {
+            if (b->up_pending[up]) sync_stream(b);
+            std::memcpy(b->h_up[up], src, bytes);
+            double2* d = stage_buf<double2>(b, up == 0 ? kStS : kStV, cnt);
+            HIPCHK(hipMemcpyAsync(d, b->h_up[up], bytes, hipMemcpyHostToDevice, st));
+            b->up_pending[up] = true;
+            dsrc = d;
+        } else {
+            tmp = dalloc<double2>(cnt);
+            HIPCHK(hipMemcpyAsync(tmp, src, bytes, hipMemcpyHostToDevice, st));
+            dsrc = tmp;
+        }
     }
     const long long total = static_cast<long long>(rows) * m;
     k_rows_to_tiles<double2><<<blocks_for(total, 256), 256, 0, st>>>(dsrc, ld, rows, m, row0, dst, ld == 0 ? 1 : 0);
@@ -2607,7 +2658,16 @@ int g2g_batch_create(g2g_plan_t P, int32_t rows, int32_t precision, int32_t per_
         b->n_active = dalloc<int>(4);  // rows, tiles; a partial pass's spare pair
         b->error = dalloc<int>(1);
         HIPCHK(hipMemsetAsync(b->error, 0, sizeof(int), b->stream));
-        HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&b->h_active), 16 * sizeof(int), hipHostMallocDefault));
+        {
+            unsigned char* h = nullptr;
+            HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&h), 64 + 2 * kPinnedUpload + rp * 16, hipHostMallocDefault));
+            b->h_active = reinterpret_cast<int*>(h);
+            b->h_up[0] = h + 64;
+            b->h_up[1] = b->h_up[0] + kPinnedUpload;
+            b->h_res = reinterpret_cast<double*>(b->h_up[1] + kPinnedUpload);
+            b->h_status = reinterpret_cast<int*>(b->h_res + rp);
+            b->h_iters = b->h_status + rp;
+        }
         k_fill_int<<<blocks_for(rp, 256), 256, 0, b->stream>>>(b->status, kNotSimulated, rp);
         k_fill_int<<<blocks_for(rp, 256), 256, 0, b->stream>>>(b->iters, 0, rp);
         HIPCHK(hipGetLastError());
@@ -2624,7 +2684,7 @@ int g2g_batch_set_v(g2g_batch_t b, const double* V, int64_t ld, int32_t rows, in
         if (!b || !V) throw std::invalid_argument("null argument");
         check_rows(b, rows, row0);
         const int n = b->plan->nr.n;
-        to_tiles(V, ld, rows, n, row0, on_device, b->V, b->stream);
+        to_tiles(b, 1, V, ld, rows, n, row0, on_device, b->V);
         b->v_bcast = ld == 0 && row0 == 0 && rows == b->rows;
         if (b->v_bcast) {  // keep the one row (a later warm solve's fallback start)
             if (!b->v_row) b->v_row = dalloc<double2>(static_cast<size_t>(n));
@@ -2640,7 +2700,7 @@ int g2g_batch_set_sbus(g2g_batch_t b, const double* S, int64_t ld, int32_t rows,
     return guarded([&] {
         if (!b || !S) throw std::invalid_argument("null argument");
         check_rows(b, rows, row0);
-        to_tiles(S, ld, rows, b->plan->nr.n, row0, on_device, b->S, b->stream);
+        to_tiles(b, 0, S, ld, rows, b->plan->nr.n, row0, on_device, b->S);
     });
 }
 
@@ -2791,6 +2851,12 @@ int g2g_batch_branch_flows(g2g_batch_t b, int32_t m, const int32_t* from, const 
             if (from[l] < -1 || from[l] >= n || to[l] < -1 || to[l] >= n)
                 throw std::invalid_argument("branch bus out of range");
         const int rows = b->active_rows;
+        const int n_trip = trip_ptr && trip_branch ? trip_ptr[rows] : 0;
+        for (int r = 0; n_trip > 0 && r < rows; ++r)
+            if (trip_ptr[r + 1] < trip_ptr[r]) throw std::invalid_argument("trip_ptr is not monotone");
+        for (int q = n_trip > 0 ? trip_ptr[0] : 0; q < n_trip; ++q)
+            if (trip_branch[q] < 0 || trip_branch[q] >= m) throw std::invalid_argument("tripped branch out of range");
+        if (rows <= 0) return;
         const int T = (rows + kLanes - 1) / kLanes;
         DeviceScratch s;
         int* d_f = s.get<int>(m);
@@ -2798,37 +2864,39 @@ int g2g_batch_branch_flows(g2g_batch_t b, int32_t m, const int32_t* from, const 
         double2* d_y = s.get<double2>(4 * static_cast<size_t>(m));
         double* d_bo = s.get<double>(m);
         double* d_be = s.get<double>(m);
-        const size_t cnt = static_cast<size_t>(T) * m * kLanes;
-        double* d_or = s.get<double>(cnt);
-        double* d_ex = s.get<double>(cnt);
+        // device outputs are written in place, host ones through a device copy
+        auto device = [](const void* p) {
+            hipPointerAttribute_t at{};
+            const hipError_t e = hipPointerGetAttributes(&at, p);
+            if (e != hipSuccess) (void)hipGetLastError();  // plain host memory
+            return e == hipSuccess && at.type == hipMemoryTypeDevice;
+        };
+        const size_t cnt = static_cast<size_t>(rows) * m;
+        const bool dor = device(or_amps), dex = device(ex_amps);
+        double* d_or = dor ? or_amps : s.get<double>(cnt);
+        double* d_ex = dex ? ex_amps : s.get<double>(cnt);
         hipStream_t st = b->stream;
         HIPCHK(hipMemcpyAsync(d_f, from, m * sizeof(int), hipMemcpyHostToDevice, st));
         HIPCHK(hipMemcpyAsync(d_t, to, m * sizeof(int), hipMemcpyHostToDevice, st));
         HIPCHK(hipMemcpyAsync(d_y, y4, 4 * static_cast<size_t>(m) * sizeof(double2), hipMemcpyHostToDevice, st));
         HIPCHK(hipMemcpyAsync(d_bo, base_or, m * sizeof(double), hipMemcpyHostToDevice, st));
         HIPCHK(hipMemcpyAsync(d_be, base_ex, m * sizeof(double), hipMemcpyHostToDevice, st));
-        k_branch_flows<<<blocks_for(static_cast<long long>(cnt), 256), 256, 0, st>>>(
-            b->V, n, d_f, d_t, d_y, d_bo, d_be, m, T, d_or, d_ex);
+        const dim3 grid((m + kFlowBranches - 1) / kFlowBranches, T);
+        k_branch_flows<<<grid, 256, 0, st>>>(b->V, n, d_f, d_t, d_y, d_bo, d_be, m, rows, d_or, d_ex);
         HIPCHK(hipGetLastError());
-        std::vector<double> ho(cnt), he(cnt);
-        HIPCHK(hipMemcpyAsync(ho.data(), d_or, cnt * sizeof(double), hipMemcpyDeviceToHost, st));
-        HIPCHK(hipMemcpyAsync(he.data(), d_ex, cnt * sizeof(double), hipMemcpyDeviceToHost, st));
+        if (n_trip > 0) {
+            int* d_tp = s.get<int>(static_cast<size_t>(rows) + 1);
+            int* d_tb = s.get<int>(static_cast<size_t>(n_trip));
+            HIPCHK(hipMemcpyAsync(d_tp, trip_ptr, (static_cast<size_t>(rows) + 1) * sizeof(int), hipMemcpyHostToDevice,
+                                  st));
+            HIPCHK(hipMemcpyAsync(d_tb, trip_branch, static_cast<size_t>(n_trip) * sizeof(int), hipMemcpyHostToDevice,
+                                  st));
+            k_trip_flows<<<blocks_for(rows, 256), 256, 0, st>>>(d_tp, d_tb, rows, m, d_or, d_ex);
+            HIPCHK(hipGetLastError());
+        }
+        if (!dor) HIPCHK(hipMemcpyAsync(or_amps, d_or, cnt * sizeof(double), hipMemcpyDeviceToHost, st));
+        if (!dex) HIPCHK(hipMemcpyAsync(ex_amps, d_ex, cnt * sizeof(double), hipMemcpyDeviceToHost, st));
         HIPCHK(hipStreamSynchronize(st));
-        for (int r = 0; r < rows; ++r)
-            for (int l = 0; l < m; ++l) {
-                const size_t i = (static_cast<size_t>(r / kLanes) * m + l) * kLanes + (r % kLanes);
-                or_amps[static_cast<size_t>(r) * m + l] = ho[i];
-                ex_amps[static_cast<size_t>(r) * m + l] = he[i];
-            }
-        // tripped branches carry no current
-        if (trip_ptr && trip_branch)
-            for (int r = 0; r < rows; ++r)
-                for (int q = trip_ptr[r]; q < trip_ptr[r + 1]; ++q) {
-                    const int l = trip_branch[q];
-                    if (l < 0 || l >= m) throw std::invalid_argument("tripped branch out of range");
-                    or_amps[static_cast<size_t>(r) * m + l] = 0.0;
-                    ex_amps[static_cast<size_t>(r) * m + l] = 0.0;
-                }
     });
 }
 
@@ -2989,14 +3057,18 @@ int g2g_batch_get_results(g2g_batch_t b, int32_t* status, int32_t* iters, double
 {
     return guarded([&] {
         if (!b) throw std::invalid_argument("null batch");
-        HIPCHK(hipStreamSynchronize(b->stream));
         const size_t r = static_cast<size_t>(b->rows);
-        if (status) HIPCHK(hipMemcpy(status, b->status, r * sizeof(int), hipMemcpyDeviceToHost));
-        if (iters) HIPCHK(hipMemcpy(iters, b->iters, r * sizeof(int), hipMemcpyDeviceToHost));
-        if (residual) HIPCHK(hipMemcpy(residual, b->res, r * sizeof(double), hipMemcpyDeviceToHost));
+        // one wait for all three
+        hipStream_t st = b->stream;
+        if (status) HIPCHK(hipMemcpyAsync(b->h_status, b->status, r * sizeof(int), hipMemcpyDeviceToHost, st));
+        if (iters) HIPCHK(hipMemcpyAsync(b->h_iters, b->iters, r * sizeof(int), hipMemcpyDeviceToHost, st));
+        if (residual) HIPCHK(hipMemcpyAsync(b->h_res, b->res, r * sizeof(double), hipMemcpyDeviceToHost, st));
+        sync_stream(b);
+        if (status) std::memcpy(status, b->h_status, r * sizeof(int));
+        if (iters) std::memcpy(iters, b->h_iters, r * sizeof(int));
+        if (residual) std::memcpy(residual, b->h_res, r * sizeof(double));
     });
 }
-
 int g2g_batch_eval(g2g_batch_t b, double* F, double* J, double* residual)
 {
     return guarded([&] {

@@ -100,6 +100,8 @@ struct ExtArgs {
     int part_stride, splits;
 };
 
+constexpr int kFlowBranches = 32;  // branches of a k_branch_flows workgroup
+
 // limit-violation check of solved rows (one wavefront per row)
 struct ViolationArgs {
     const double2* V;           // [T][n][64]

@@ -2032,6 +2032,17 @@ __global__ void k_fill_int(int* __restrict__ p, int v, long long n)
 }
 
 // tile_active[t] = rows of tile t still iterating
+// a solve's start: rows [0, active) iterate, the others are not simulated
+__global__ void k_init_rows(int active, int rows_pad, int* __restrict__ status, int* __restrict__ iters,
+                            int* __restrict__ tile_active)
+{
+    const int r = blockIdx.x * blockDim.x + threadIdx.x;
+    if (r >= rows_pad) return;
+    status[r] = r < active ? kActive : kNotSimulated;
+    iters[r] = 0;
+    if (r % kLanes == 0) tile_active[r / kLanes] = min(max(active - r, 0), kLanes);
+}
+
 __global__ void k_count_tiles(const int* __restrict__ status, int rows_pad, int* __restrict__ tile_active)
 {
     const int t = blockIdx.x;
@@ -2074,33 +2085,60 @@ __global__ void k_move_vals(const T* __restrict__ src, T* __restrict__ dst, cons
 //   I_or = yff V_f + yft V_t,  I_ex = ytf V_f + ytt V_t,  amps = |I| * base current
 // One thread per (tile, branch, lane); outputs tiled [T][m][64].  A side with
 // bus -1 (no terminal) reports 0.
-__global__ void k_branch_flows(const double2* __restrict__ V, int n, const int* __restrict__ from,
-                               const int* __restrict__ to, const double2* __restrict__ y4,
-                               const double* __restrict__ base_or, const double* __restrict__ base_ex, int m,
-                               int T, double* __restrict__ or_t, double* __restrict__ ex_t)
+// Rows x m outputs, row-major: a workgroup computes a tile's 64 rows of
+// kFlowBranches branches with a lane per row (the tiled V's coalesced reads)
+// and writes them through LDS with a lane per branch, so the caller's layout
+// needs no transposition on the host (2,718 rows x 3,000 branches: about 50 ms
+// of strided host copies).  Bound by the output's writes.
+__global__ __launch_bounds__(256) void k_branch_flows(const double2* __restrict__ V, int n,
+                                                      const int* __restrict__ from, const int* __restrict__ to,
+                                                      const double2* __restrict__ y4,
+                                                      const double* __restrict__ base_or,
+                                                      const double* __restrict__ base_ex, int m, int rows,
+                                                      double* __restrict__ or_amps, double* __restrict__ ex_amps)
 {
-    const long long gid = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (gid >= static_cast<long long>(T) * m * kLanes) return;
-    const int lane = static_cast<int>(gid & (kLanes - 1));
-    const long long tl = gid / kLanes;
-    const int l = static_cast<int>(tl % m);
-    const size_t tile = static_cast<size_t>(tl / m);
-    const int f = from[l], t = to[l];
-    const double2 z = make_double2(0.0, 0.0);
-    const double2 vf = f >= 0 ? V[tidx(tile, n, f, lane)] : z;
-    const double2 vt = t >= 0 ? V[tidx(tile, n, t, lane)] : z;
-    const double2* y = y4 + 4 * static_cast<size_t>(l);
-    double2 io = z, ie = z;
-    if (f >= 0) {
-        const double2 a = cmul(y[0], vf), b = cmul(y[1], vt);
-        io = make_double2(a.x + b.x, a.y + b.y);
+    __shared__ double so[kFlowBranches][kLanes + 1], se[kFlowBranches][kLanes + 1];
+    const int lane = threadIdx.x & (kLanes - 1), wave = threadIdx.x / kLanes;
+    const int l0 = blockIdx.x * kFlowBranches;
+    const size_t tile = blockIdx.y;
+    for (int q = wave; q < kFlowBranches && l0 + q < m; q += 256 / kLanes) {
+        const int l = l0 + q, f = from[l], t = to[l];
+        const double2 z = make_double2(0.0, 0.0);
+        const double2 vf = f >= 0 ? V[tidx(tile, n, f, lane)] : z;
+        const double2 vt = t >= 0 ? V[tidx(tile, n, t, lane)] : z;
+        const double2* y = y4 + 4 * static_cast<size_t>(l);
+        double2 io = z, ie = z;
+        if (f >= 0) {
+            const double2 a = cmul(y[0], vf), b = cmul(y[1], vt);
+            io = make_double2(a.x + b.x, a.y + b.y);
+        }
+        if (t >= 0) {
+            const double2 a = cmul(y[2], vf), b = cmul(y[3], vt);
+            ie = make_double2(a.x + b.x, a.y + b.y);
+        }
+        so[q][lane] = sqrt(fma(io.x, io.x, io.y * io.y)) * base_or[l];
+        se[q][lane] = sqrt(fma(ie.x, ie.x, ie.y * ie.y)) * base_ex[l];
     }
-    if (t >= 0) {
-        const double2 a = cmul(y[2], vf), b = cmul(y[3], vt);
-        ie = make_double2(a.x + b.x, a.y + b.y);
+    __syncthreads();
+    for (int i = threadIdx.x; i < kFlowBranches * kLanes; i += 256) {
+        const int q = i % kFlowBranches, r = i / kFlowBranches;
+        const size_t row = tile * kLanes + r;
+        if (l0 + q >= m || row >= static_cast<size_t>(rows)) continue;
+        or_amps[row * m + l0 + q] = so[q][r];
+        ex_amps[row * m + l0 + q] = se[q][r];
     }
-    or_t[gid] = sqrt(fma(io.x, io.x, io.y * io.y)) * base_or[l];
-    ex_t[gid] = sqrt(fma(ie.x, ie.x, ie.y * ie.y)) * base_ex[l];
+}
+
+// tripped branches carry no current
+__global__ void k_trip_flows(const int* __restrict__ trip_ptr, const int* __restrict__ trip, int rows, int m,
+                             double* __restrict__ or_amps, double* __restrict__ ex_amps)
+{
+    const int row = blockIdx.x * blockDim.x + threadIdx.x;
+    if (row >= rows) return;
+    for (int q = trip_ptr[row]; q < trip_ptr[row + 1]; ++q) {
+        or_amps[static_cast<size_t>(row) * m + trip[q]] = 0.0;
+        ex_amps[static_cast<size_t>(row) * m + trip[q]] = 0.0;
+    }
 }
 
 // ---------------------------------------------------------------------------

@@ -278,7 +278,7 @@ int g2g_batch_warm_start(g2g_batch_t batch, g2g_mlp_t mlp, const uint8_t *mask, 
  * (sqrt(3) vn_kv 1e3)).  y4 holds 4 m complex values per branch in the order
  * yff, yft, ytf, ytt; a bus of -1 marks a missing terminal (0 A).  Row r's
  * tripped branches trip_branch[trip_ptr[r] .. trip_ptr[r+1]) report 0
- * (trip_ptr / trip_branch nullable).  Outputs rows x m, host arrays. */
+ * (trip_ptr / trip_branch nullable).  Outputs rows x m, host or device arrays. */
 int g2g_batch_branch_flows(g2g_batch_t batch, int32_t m, const int32_t *from, const int32_t *to, const double *y4,
                            const double *base_or, const double *base_ex, const int32_t *trip_ptr,
                            const int32_t *trip_branch, double *or_amps, double *ex_amps);

@@ -1,0 +1,55 @@
+"""Branch currents at the edges of the flow kernel's tiles (64 rows x 32
+branches): ragged rows and branch counts, missing terminals, tripped branches,
+host and device outputs, against the closed form."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from gpusim2grid_amd import _capi
+from gpusim2grid_amd import synthetic as syn
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,m,rows", [(14, 1, 1), (14, 20, 64), (118, 33, 65), (118, 180, 130), (118, 32, 63)])
+def test_flows_match_the_closed_form(n, m, rows):
+    import torch
+    g = {14: syn.grid_c0, 118: syn.grid_118}[n]()
+    rng = np.random.default_rng(n + m + rows)
+    V = (1.0 + 0.05 * rng.standard_normal((rows, n))) * np.exp(0.3j * rng.standard_normal((rows, n)))
+    B = _capi.Batch(_capi.Plan.from_grid(g.Ybus, g.pv, g.pq, g.slack), rows)
+    B.set_v(V)
+    f, t = g.branch_from[:m].copy(), g.branch_to[:m].copy()
+    if m > 2:
+        f[1], t[2] = -1, -1  # missing terminals
+    y = [a[:m] for a in (g.yff, g.yft, g.ytf, g.ytt)]
+    bo, be = rng.uniform(1, 2, m), rng.uniform(1, 2, m)
+    trips = [sorted(rng.choice(m, size=min(m, r % 3), replace=False).tolist()) for r in range(rows)]
+    orr, ex = B.branch_flows(f, t, *y, bo, be, trips=trips)
+    z = np.zeros((rows, 1))
+    Vx = np.concatenate([V, z], axis=1)  # bus -1 reads 0
+    ro = np.where(f >= 0, np.abs(y[0] * Vx[:, f] + y[1] * Vx[:, t]) * bo, 0.0)
+    re = np.where(t >= 0, np.abs(y[2] * Vx[:, f] + y[3] * Vx[:, t]) * be, 0.0)
+    for r, tr in enumerate(trips):
+        ro[r, tr] = re[r, tr] = 0.0
+    # a few FP64 roundings of terms of this size
+    scale = 1e-14 * (np.abs(y[0]).max() + np.abs(y[1]).max()) * 4
+    assert np.abs(orr - ro).max() < scale and np.abs(ex - re).max() < scale
+    # the same into device arrays
+    do, de = (torch.full((rows, m), -1.0, dtype=torch.float64, device="cuda") for _ in range(2))
+    torch.cuda.synchronize()
+    y4 = np.ascontiguousarray(np.stack(y, axis=1), dtype=np.complex128)
+    tp = np.concatenate([[0], np.cumsum([len(x) for x in trips])]).astype(np.int32)
+    tb = np.array([b for x in trips for b in x] + [0], np.int32)
+    f, t = f.astype(np.int32), t.astype(np.int32)
+    P = lambda a: a.ctypes.data_as(ctypes.c_void_p)  # noqa: E731
+    assert _capi.lib().g2g_batch_branch_flows(B._h, m, P(f), P(t), P(y4), P(bo), P(be), P(tp), P(tb),
+                                              ctypes.c_void_p(do.data_ptr()), ctypes.c_void_p(de.data_ptr())) == 0
+    np.testing.assert_array_equal(do.cpu().numpy(), orr)
+    np.testing.assert_array_equal(de.cpu().numpy(), ex)
+    bad = np.array([m] * tb.size, np.int32)  # a branch out of range is still refused
+    if tp[-1] > 0:
+        assert _capi.lib().g2g_batch_branch_flows(B._h, m, P(f), P(t), P(y4), P(bo), P(be), P(tp), P(bad),
+                                                  ctypes.c_void_p(do.data_ptr()),
+                                                  ctypes.c_void_p(de.data_ptr())) == _capi.G2G_ERR_INVALID
