@@ -1484,18 +1484,24 @@ RowShape row_shape(const g2g_batch_s* b, int R)
     const size_t all = static_cast<size_t>(r.n_blk) * 4 * sizeof(Real);
     const size_t with_v = row_lds_bytes<Real>(r.n, r.nb, true, ed), no_v = row_lds_bytes<Real>(r.n, r.nb, false, ed);
     // threads: enough that the widest levels are a few records a thread (997
-    // buses FP64, 12,288 rows: 512 threads 10.4 ms, 256 11.7; 2,000 mixed, 8,192
-    // rows: 1,024 6.8 ms, 512 7.1), few where several workgroups share a CU
+    // buses FP64, 12,288 rows: 512 threads 10.4 ms, 256 11.7; 2,000 mixed, 4,096
+    // rows: 1,024 3.02 ms, 512 3.15), few where several workgroups share a CU
     // (118 buses, 16,384 rows: 128 1.09 ms, 256 1.72)
     s.threads = r.nb <= 64 ? 64 : r.nb <= 300 ? 128 : r.nb <= 600 ? 256 : r.nb <= 1500 ? 512 : 1024;
-    if (with_v + all <= limit) {
+    // Workgroups a CU: 16 wavefronts fit its registers.  With more rows than CUs,
+    // two of 512 threads, their lowest blocks in the scratch, beat one with every
+    // block in LDS (997 buses, 777 rows: mixed 0.55 / 0.72 ms, FP64 0.78 / 0.82);
+    // one of 1,024 takes the whole LDS (6,500 mixed, 1,000 rows: 5.1 ms, half 6.1;
+    // 2,000 FP64, 777 rows: 1.42, half 1.66).
+    const int waves_fit = std::max(1, kRowMaxThreads / s.threads);
+    const size_t room = R > b->n_cu && waves_fit >= 2 && 2 * no_v <= limit ? limit / 2 : limit;
+    if (with_v + all <= room) {
         s.blk_lds = s.v_lds = true;
         s.lds = with_v + all;
-    } else if (no_v + all <= limit) {
+    } else if (no_v + all <= room) {
         s.blk_lds = true;
         s.lds = no_v + all;
     } else {
-        const size_t room = R > b->n_cu && 2 * no_v <= limit && 2 * s.threads <= 2048 ? limit / 2 : limit;
         s.v_lds = 2 * with_v <= room;
         const size_t base = s.v_lds ? with_v : no_v;
         if (base > room) return s;
@@ -1504,7 +1510,7 @@ RowShape row_shape(const g2g_batch_s* b, int R)
         s.lds = base + fit * 4 * sizeof(Real);
         while (r.lev_blk[s.lev_lds] < s.lds0) ++s.lev_lds;
     }
-    s.per_cu = std::max(1, std::min<int>(static_cast<int>(limit / s.lds), 2048 / s.threads));
+    s.per_cu = std::max(1, std::min<int>(static_cast<int>(limit / s.lds), waves_fit));
     s.scratch = row_scratch_bytes<Real>(r.n, r.nb, s.lds0, s.v_lds, b->ir_steps > 0);
     s.ok = true;
     return s;
@@ -1525,13 +1531,22 @@ bool use_rows(const g2g_batch_s* b, int active_rows)
     if (!s.ok) return false;
     const int env = rows_env();
     if (env >= 0) return env == 1;
-    // Where the two cross over, measured per solve (tile kernels / row solver):
-    // 118 buses FP64 16,384 rows 1.73 / 1.09 ms (the row solver at any count: several workgroups a CU);
-    // 997 FP64 12,288 rows 12.1 / 10.4 ms; 2,000 mixed 12,288 rows 10.6 / 10.2, 8,192 10.4 / 6.8 (one a CU);
-    // 2,000 FP64 (200 KB of scratch a workgroup, in the L2 and last-level cache) 4,096 rows 8.9 / 6.4, 8,192 15.1 / 12.9;
-    // 6,500 mixed (420 KB) 1,024 rows 7.0 / 6.2, 2,048 11.3 / 12.2; 6,500 FP64 (900 KB) 768 rows 10.1 / 7.4, 1,024 10.7 / 10.5
-    if (s.blk_lds && s.per_cu >= 4) return true;
-    return active_rows <= b->n_cu * (s.blk_lds ? 48 : s.scratch <= (256u << 10) ? 24 : s.scratch <= (512u << 10) ? 4 : 3);
+    // Where the two cross over, measured per solve (tile kernels / row solver, ms).
+    // Two workgroups a CU or more, at any count: 118 buses FP64 16,384 rows 1.66 / 0.97; 997 mixed
+    // 16,384 rows 10.4 / 6.8, 65,536 36.0 / 27.3, FP64 16,384 13.1 / 11.4, 65,536 50.8 / 45.6.
+    // One a CU, by what a row keeps in the scratch (in the L2 and last-level cache) beside the LDS:
+    //   none but V   2,000 mixed 12,288 rows 10.6 / 9.0, 14,336 11.7 / 10.5, 16,384 12.1 / 11.9
+    //   FP64         2,000 (176 KB) 8,192 rows 15.0 / 11.5, 12,288 19.0 / 17.1; 3,000 (346 KB) 4,096 14.1 / 11.4;
+    //                4,500 (598 KB) 2,048 13.0 / 9.6; 6,500 (876 KB) 768 10.1 / 7.6, 1,024 10.7 / 11.0
+    //   mixed        3,000 (116 KB) 8,192 14.0 / 13.4; 4,500 (254 KB) 4,096 10.3 / 10.9;
+    //                6,500 (409 KB) 2,048 11.3 / 9.9
+    if (s.per_cu >= 2) return true;
+    const size_t kb = s.scratch >> 10;
+    int per_cu;  // rows a CU
+    if (s.blk_lds) per_cu = 56;
+    else if (sizeof(Real) == 8) per_cu = kb <= 200 ? 48 : kb <= 400 ? 16 : kb <= 640 ? 8 : 3;
+    else per_cu = kb <= 200 ? 32 : 8;
+    return active_rows <= b->n_cu * per_cu;
 }
 
 template <typename Real, bool BL, bool VL>

@@ -198,8 +198,8 @@ RowPlan build_row_plan(const NrPlan& P)
         const int first = static_cast<int>(R.back_col.size());
         if (first >= (1 << 24)) return R;
         const auto& c = col[k];
-        R.back.insert(R.back.end(), {diag[k], first | (static_cast<int>(c.size()) << 24), c.size() > 0 ? c[0] : 0,
-                                     c.size() > 1 ? c[1] : 0});
+        R.back.insert(R.back.end(), {diag[k], first | (static_cast<int>(c.size()) << 24), c.size() > 0 ? c[0] : k,
+                                     c.size() > 1 ? c[1] : k});
         if (c.size() > 2) R.back_col.insert(R.back_col.end(), c.begin() + 2, c.end());
     }
     R.solo_f = R.solo_b = R.n_lev;

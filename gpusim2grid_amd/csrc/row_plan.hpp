@@ -45,7 +45,7 @@ struct RowPlan {
     std::vector<int> rec;        // 4 words per record
     std::vector<int> rec2;       // 2 words per record: its second term
     std::vector<int> term;       // 2 words per further term: {pivot block, term}
-    std::vector<int> back;       // 4 words per bus: {diagonal block, first | count << 24, two columns' buses}
+    std::vector<int> back;       // 4 words per bus: {diagonal block, first | count << 24, two columns' buses (itself: none)}
     std::vector<int> back_col;   // buses of a pivot's third and further off-diagonal blocks
     // levels from which on no level has more records (buses) than a wavefront has lanes
     int solo_f = 0, solo_b = 0;

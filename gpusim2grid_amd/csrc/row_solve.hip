@@ -12,8 +12,11 @@
 // host round trip.
 //
 // What bounds it: the levels' dependent chain (record, terms' blocks, target,
-// barrier), about 0.4 us a level with the blocks in LDS.  The arithmetic is
-// small (a 6,500-bus factorization is 17,785 updates of 2 x 2 blocks).
+// barrier): 2,000 buses mixed, one row, all in LDS, take 55 us an iteration,
+// half of it the factorization's 30 levels, an eighth the substitution's.  The
+// arithmetic is small (a 6,500-bus factorization is 17,785 updates of 2 x 2
+// blocks).  6,500 buses FP64 (150 us an iteration) spend a third in the
+// mismatch, whose V, tables and low blocks are in the L2.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -67,19 +70,20 @@ __device__ __forceinline__ Real clamp_pivot(Real d, Real eps)
 
 // The inverse of a diagonal block: its adjugate over its determinant, one
 // reciprocal on the levels' dependent chain; with its two pivots taken in
-// order (D0, then det / D0) where one of them is below the clamp.
+// order (D00, then det / D00) where one of them is below the clamp.  Blocks
+// are held column by column: {00, 10, 01, 11}.
 template <typename Real>
 __device__ __forceinline__ typename V4<Real>::T invert(typename V4<Real>::T D, Real eps)
 {
-    const Real det = fma(D[0], D[3], -D[1] * D[2]);
+    const Real det = fma(D[0], D[3], -D[2] * D[1]);
     const Real i = inv_of(det);
     typename V4<Real>::T R = {D[3] * i, -D[1] * i, -D[2] * i, D[0] * i};
     if (fabs(D[0]) < eps || fabs(det) < eps * fabs(D[0])) {
         const Real i1 = inv_of(clamp_pivot(D[0], eps));
-        const Real l = D[2] * i1;
-        const Real i2 = inv_of(clamp_pivot(fma(-l, D[1], D[3]), eps));
-        const Real u = i1 * D[1] * i2;
-        R = typename V4<Real>::T{fma(u, l, i1), -u, -i2 * l, i2};
+        const Real l = D[1] * i1;
+        const Real i2 = inv_of(clamp_pivot(fma(-l, D[2], D[3]), eps));
+        const Real u = i1 * D[2] * i2;
+        R = typename V4<Real>::T{fma(u, l, i1), -i2 * l, -u, i2};
     }
     return R;
 }
@@ -119,8 +123,8 @@ __global__ __launch_bounds__(kRowMaxThreads) void k_row_solve(RowArgs<Real> a)
         at += row_align(bytes);
         return p;
     };
-    double* red = reinterpret_cast<double*>(take(2 * 16 * sizeof(double) + sizeof(int)));
-    int* slice_next = reinterpret_cast<int*>(red + 32);
+    auto* red = reinterpret_cast<unsigned long long*>(take(kRowRedBytes));
+    int* slice_next = reinterpret_cast<int*>(red + 4);
     Real* b = reinterpret_cast<Real*>(take(static_cast<size_t>(a.nb) * 2 * sizeof(Real)));
     R2* b2 = reinterpret_cast<R2*>(b);
     const bool edits = a.ed.n_ed != nullptr;
@@ -232,7 +236,11 @@ __global__ __launch_bounds__(kRowMaxThreads) void k_row_solve(RowArgs<Real> a)
         bool decide = !a.skip_first;
         int iter = a.clock ? *a.clock + a.iter0 : a.iter0, st = kActive, n_upd = 0;
         double jm = 0.0;
-        if (tid == 0) *slice_next = n_wave;
+        int turn = 0;
+        if (tid == 0) {
+            *slice_next = n_wave;
+            red[0] = red[1] = 0ull;
+        }
         __syncthreads();
 
         // a Ybus value less the row's edits of entry k
@@ -244,34 +252,33 @@ __global__ __launch_bounds__(kRowMaxThreads) void k_row_solve(RowArgs<Real> a)
                 }
             return y;
         };
-        // one record: a block's (blocks) or a right-hand side's updates by a
-        // level's pivots; a right-hand side is taken as a block of one column
+        // One record: a block's (blocks) or a right-hand side's updates by a
+        // level's pivots.  A right-hand side is run as a block whose two
+        // columns are both the vector: the same loads, arithmetic and stores
+        // (its two stores write one value to one place), so a wavefront of
+        // mixed records has no divergent path, and all its LDS reads go out
+        // together (under a condition each path's would be waited for where
+        // the paths join).  A solve so, against a branch for each kind: 118 FP64
+        // 4,096 rows 0.28 / 0.30 ms; 2,000 mixed 777 rows 0.80 / 0.90.
         auto update = [&](auto in, const int4 rec, const int2 rec2, Real eps, bool blocks) {
             const int tgt = rec.x & (kRowRhs - 1), cnt = rec.y >> 24, first = rec.y & 0xFFFFFF;
             const bool rhs = rec.x & kRowRhs;
             if (!rhs && !blocks) return;
-            B4 t;
-            if (rhs) {
-                const R2 y = b2[tgt];
-                t = B4{y[0], Real(0), y[1], Real(0)};
-            } else {
-                t = *blk(in, tgt);
-            }
+            auto column = [&](int q) { return rhs ? b2 + q : reinterpret_cast<R2*>(blk(in, rhs ? 0 : q)); };
+            const int second = rhs ? 0 : 1;
+            R2* const p0 = column(tgt);
+            R2* const p1 = p0 + second;
+            R2 t0 = *p0, t1 = *p1;
             auto term = [&](int d, int w) {
+                const R2* u = column(rhs ? w >> 8 : d + (w >> 8));
                 const B4 L = *blk(in, d + (w & 0xFF)), D = *blk(in, d);
-                B4 U;
-                if (rhs) {
-                    const R2 y = b2[w >> 8];
-                    U = B4{y[0], Real(0), y[1], Real(0)};
-                } else {
-                    U = *blk(in, d + (w >> 8));
-                }
-                const Real w00 = fma(D[0], U[0], D[1] * U[2]), w01 = fma(D[0], U[1], D[1] * U[3]);
-                const Real w10 = fma(D[2], U[0], D[3] * U[2]), w11 = fma(D[2], U[1], D[3] * U[3]);
-                t[0] = fma(-L[0], w00, fma(-L[1], w10, t[0]));
-                t[1] = fma(-L[0], w01, fma(-L[1], w11, t[1]));
-                t[2] = fma(-L[2], w00, fma(-L[3], w10, t[2]));
-                t[3] = fma(-L[2], w01, fma(-L[3], w11, t[3]));
+                const R2 u0 = u[0], u1 = u[second];
+                const Real w00 = fma(D[0], u0[0], D[2] * u0[1]), w01 = fma(D[0], u1[0], D[2] * u1[1]);
+                const Real w10 = fma(D[1], u0[0], D[3] * u0[1]), w11 = fma(D[1], u1[0], D[3] * u1[1]);
+                t0[0] = fma(-L[0], w00, fma(-L[2], w10, t0[0]));
+                t1[0] = fma(-L[0], w01, fma(-L[2], w11, t1[0]));
+                t0[1] = fma(-L[1], w00, fma(-L[3], w10, t0[1]));
+                t1[1] = fma(-L[1], w01, fma(-L[3], w11, t1[1]));
             };
             term(rec.z, rec.w);
             if (cnt > 1) {
@@ -281,14 +288,13 @@ __global__ __launch_bounds__(kRowMaxThreads) void k_row_solve(RowArgs<Real> a)
                     term(tm.x, tm.y);
                 }
             }
-            if (rhs) {
-                R2 y;
-                y[0] = t[0];
-                y[1] = t[2];
-                b2[tgt] = y;
-            } else {
-                *blk(in, tgt) = (rec.x & kRowInvert) ? invert<Real>(t, eps) : t;
+            if (rec.x & kRowInvert) {
+                const B4 v = invert<Real>(B4{t0[0], t0[1], t1[0], t1[1]}, eps);
+                t0 = R2{v[0], v[1]};
+                t1 = R2{v[2], v[3]};
             }
+            *p0 = t0;
+            *p1 = t1;
         };
         // factorization and forward substitution (blocks), or the latter alone:
         // the wide levels by every thread with a barrier after each, the
@@ -343,22 +349,26 @@ __global__ __launch_bounds__(kRowMaxThreads) void k_row_solve(RowArgs<Real> a)
         };
         // x over b, level by level from the top: the narrow levels by one
         // wavefront, the wide ones by every thread
+        // (the first two columns' reads go out with the pivot's; a missing
+        // column reads the pivot's own block, times zero)
         auto solve_bus = [&](auto in, int k, const int4 r) {
             const int c = r.y >> 24, first = r.y & 0xFFFFFF;
-            const B4 D = *blk(in, r.x);
             R2 t = b2[k];
-            auto sub = [&](int q, int j) {
-                const B4 U = *blk(in, r.x + 2 + 2 * q);
-                const R2 x = b2[j];
-                t[0] = fma(-U[0], x[0], fma(-U[1], x[1], t[0]));
-                t[1] = fma(-U[2], x[0], fma(-U[3], x[1], t[1]));
+            const B4 D = *blk(in, r.x);
+            const B4 U0 = *blk(in, c > 0 ? r.x + 2 : r.x), U1 = *blk(in, c > 1 ? r.x + 4 : r.x);
+            R2 x0 = b2[r.z], x1 = b2[r.w];
+            if (c < 1) x0 = R2{Real(0), Real(0)};
+            if (c < 2) x1 = R2{Real(0), Real(0)};
+            auto sub = [&](const B4& U, const R2& x) {
+                t[0] = fma(-U[0], x[0], fma(-U[2], x[1], t[0]));
+                t[1] = fma(-U[1], x[0], fma(-U[3], x[1], t[1]));
             };
-            if (c > 0) sub(0, r.z);
-            if (c > 1) sub(1, r.w);
-            for (int q = 2; q < c; ++q) sub(q, a.back_col[first + q - 2]);
+            sub(U0, x0);
+            sub(U1, x1);
+            for (int q = 2; q < c; ++q) sub(*blk(in, r.x + 2 + 2 * q), b2[a.back_col[first + q - 2]]);
             R2 x;
-            x[0] = fma(D[0], t[0], D[1] * t[1]);
-            x[1] = fma(D[2], t[0], D[3] * t[1]);
+            x[0] = fma(D[0], t[0], D[2] * t[1]);
+            x[1] = fma(D[1], t[0], D[3] * t[1]);
             b2[k] = x;
         };
         auto substitute = [&]() {
@@ -442,7 +452,7 @@ __global__ __launch_bounds__(kRowMaxThreads) void k_row_solve(RowArgs<Real> a)
                         const double2 w = mulc(vi, t);
                         const Real wx = static_cast<Real>(w.x), wy = static_cast<Real>(w.y);
                         const bool rq = en[g].y & 1, cq = en[g].y & 2;
-                        store(en[g].y >> 2, B4{wy, cq ? wx : Real(0), rq ? -wx : Real(0), rq && cq ? wy : Real(0)});
+                        store(en[g].y >> 2, B4{wy, rq ? -wx : Real(0), cq ? wx : Real(0), rq && cq ? wy : Real(0)});
                         jmax = fmax(jmax, fmax(fabs(w.x), fabs(w.y)));
                     }
                 }
@@ -455,26 +465,31 @@ __global__ __launch_bounds__(kRowMaxThreads) void k_row_solve(RowArgs<Real> a)
                     const double2 z = mulc(vi, make_double2(I.x - t0.x, I.y - t0.y));
                     const double2 u = mulc(vi, make_double2(I.x + t0.x, I.y + t0.y));
                     jmax = fmax(jmax, fmax(fmax(fabs(z.x), fabs(z.y)), fmax(fabs(u.x), fabs(u.y))));
-                    store(sb.y & 0x7FFFFFFF, q ? B4{static_cast<Real>(-z.y), static_cast<Real>(u.x),
-                                                    static_cast<Real>(z.x), static_cast<Real>(u.y)}
+                    store(sb.y & 0x7FFFFFFF, q ? B4{static_cast<Real>(-z.y), static_cast<Real>(z.x),
+                                                    static_cast<Real>(u.x), static_cast<Real>(u.y)}
                                                : B4{static_cast<Real>(-z.y), Real(0), Real(0), Real(1)});
                 }
             }
+            // the workgroup's maxima: of magnitudes, whose bit patterns order as
+            // unsigned numbers with NaN above all (a NaN anywhere makes r NaN).
+            // Two sets of cells take turns: one is cleared while the other is read.
+            auto bits = [](double v) { return static_cast<unsigned long long>(__double_as_longlong(v)); };
             for (int o = 32; o > 0; o >>= 1) {
                 rmax = nan_max(rmax, __shfl_xor(rmax, o, 64));
                 jmax = fmax(jmax, __shfl_xor(jmax, o, 64));
             }
+            unsigned long long* const cell = red + turn;
             if (lane == 0) {
-                red[wave] = rmax;
-                red[16 + wave] = jmax;
+                atomicMax(cell, bits(rmax));
+                atomicMax(cell + 1, bits(jmax));
             }
             __syncthreads();
-            if (tid == 0) *slice_next = n_wave;
-            double r = red[0];
-            jm = red[16];
-            for (int w = 1; w < n_wave; ++w) {
-                r = nan_max(r, red[w]);
-                jm = fmax(jm, red[16 + w]);
+            const double r = __longlong_as_double(static_cast<long long>(cell[0]));
+            jm = __longlong_as_double(static_cast<long long>(cell[1]));
+            turn ^= 2;
+            if (tid == 0) {
+                *slice_next = n_wave;
+                red[turn] = red[turn + 1] = 0ull;
             }
             // the status rule (kernels.hip mis_status)
             const int it = iter - it0;

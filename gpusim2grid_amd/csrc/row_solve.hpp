@@ -9,6 +9,7 @@ namespace g2g {
 
 constexpr int kRowMaxEdits = 64;   // a row's Ybus edits kept in LDS
 constexpr int kRowMaxThreads = 1024;
+constexpr int kRowRedBytes = 4 * 8 + 4;  // the workgroup's maxima (two sets of two) and the next slice
 // A row that ends unconverged with a residual above this (or not finite) is
 // left as it came, for the tile kernels to finish: the iterates of a row that
 // does not contract amplify rounding, so its last one is the solver's own, and
@@ -76,7 +77,7 @@ constexpr size_t row_align(size_t v) { return (v + 31) / 32 * 32; }
 template <typename Real>
 size_t row_lds_bytes(int n, int nb, bool v_lds, bool edits)
 {
-    size_t s = row_align(2 * 16 * sizeof(double) + sizeof(int)) + row_align(static_cast<size_t>(nb) * 2 * sizeof(Real));
+    size_t s = row_align(kRowRedBytes) + row_align(static_cast<size_t>(nb) * 2 * sizeof(Real));
     if (v_lds) s += row_align(static_cast<size_t>(n) * sizeof(double2));
     if (edits)
         s += row_align(kRowMaxEdits * sizeof(double2)) + row_align(kRowMaxEdits * sizeof(int)) +
