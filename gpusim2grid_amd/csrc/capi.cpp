@@ -753,30 +753,50 @@ size_t split_backward_lds(const SymbolicLU& s)
 // The split walk's factorization: the fine sets, then the middle parts, then
 // the top part, one launch each over the first T tiles.  clamped counts are
 // added per row, so they start at zero.
+template <typename Real, int MODE>
+void launch_factor_split_mode(const g2g_plan_s* P, FactorArgs<Real> a, size_t lds, int T, hipStream_t st)
+{
+    const SymbolicLU& s = P->lu();
+    HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_factor<Real, 1, true, 0, MODE>),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
+    const int levels[3][2] = {{0, s.split_fine}, {s.split_fine, s.split_mid}, {s.split_fine + s.split_mid, 1}};
+    for (const auto& lv : levels) {
+        if (lv[1] <= 0) continue;
+        a.seg0 = lv[0];
+        k_factor<Real, 1, true, 0, MODE><<<T * lv[1], kLanes * (2 + kSplitProducers), lds, st>>>(a);
+        HIPCHK(hipGetLastError());
+    }
+}
+
+// (mode, Lw: as launch_factor's)
 template <typename Real>
 void launch_factor_split(const g2g_plan_s* P, const Real* A, Real* U, int a_stride, int u_stride,
                          const int* tile_active, const double* jmax, int* clamped, int* error, int rows, int T,
-                         double eps, Real* pend, hipStream_t st)
+                         double eps, Real* pend, hipStream_t st, int mode = kFactorFull, Real* Lw = nullptr)
 {
     const SymbolicLU& s = P->lu();
     const size_t lds = split_factor_lds<Real>(s);
     if (lds > lds_limit()) throw std::runtime_error("split factorization needs " + std::to_string(lds) + " bytes of LDS");
+    if (mode == kForwardOnly) clamped = nullptr;  // no pivots: the factorization's counts stay
     if (clamped) {
         k_fill_int<<<blocks_for(static_cast<long long>(T) * kLanes, 256), 256, 0, st>>>(clamped, 0,
                                                                                        static_cast<long long>(T) * kLanes);
         HIPCHK(hipGetLastError());
     }
-    HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_factor<Real, 1, true, 0, kFactorFull>),
-                               hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
-    const int levels[3][2] = {{0, s.split_fine}, {s.split_fine, s.split_mid}, {s.split_fine + s.split_mid, 1}};
-    for (const auto& lv : levels) {
-        if (lv[1] <= 0) continue;
-        FactorArgs<Real> a{A,   U,        P->d_prog_fs, tile_active, jmax, clamped, error, s.d, a_stride,
-                           u_stride, P->prog_fs_stride, s.slots_fs, rows, s.max_c, eps, P->d_split_seg,
-                           T,   lv[0],    pend,         s.pend_len};
-        k_factor<Real, 1, true, 0, kFactorFull><<<T * lv[1], kLanes * (2 + kSplitProducers), lds, st>>>(a);
-        HIPCHK(hipGetLastError());
+    FactorArgs<Real> a{A,   U,        P->d_prog_fs, tile_active, jmax, clamped, error, s.d, a_stride,
+                       u_stride, P->prog_fs_stride, s.slots_fs, rows, s.max_c, eps, P->d_split_seg,
+                       T,   0,        pend,         s.pend_len};
+    if constexpr (sizeof(Real) == 4) {
+        if (mode == kFactorStoreL) {
+            if (!Lw) throw std::logic_error("a multiplier-storing factorization needs its stream");
+            a.Lw = Lw;
+            return launch_factor_split_mode<Real, kFactorStoreL>(P, a, lds, T, st);
+        }
+        if (mode == kForwardOnly) return launch_factor_split_mode<Real, kForwardOnly>(P, a, lds, T, st);
+    } else {
+        if (mode != kFactorFull) throw std::logic_error("stored-multiplier walks are FP32 only");
     }
+    launch_factor_split_mode<Real, kFactorFull>(P, a, lds, T, st);
 }
 
 // The split walk's backward substitution: the top part, then the middle
@@ -907,11 +927,13 @@ void ensure_edit_cap(g2g_batch_s* b, int cap, bool keep)
     b->ed_cap = cap;
 }
 
-// The walk mode of a Newton step's main-layout factorization.  With
-// FP64-residual refinement in mixed precision it stores its L multipliers in
-// the A stream, so each refinement round solves with a forward-only walk
-// instead of a second factorization (G2G_IR_REFACTOR=1: the second
-// factorization, for comparison).
+// The walk mode of a Newton step's factorization.  With FP64-residual
+// refinement in mixed precision it stores its L multipliers in a stream of
+// their own, so each refinement round solves with a forward-only walk instead
+// of a second factorization, main or split (G2G_IR_REFACTOR=1: the second
+// factorization, for comparison: 4,001 rows of 6,500 buses, on the split
+// walk, 27.3 ms a solve, with the forward walk 25.8; two rounds a step 39.3
+// and 36.1).
 template <typename Real>
 int factor_walk_mode(const g2g_batch_s* b)
 {
@@ -953,7 +975,7 @@ void refine_fp64(g2g_batch_s* b, double eps, int T)
     int splits = std::max(1, b->mis_splits);
     while (splits < 32 && 2 * splits * T <= 512) splits *= 2;
     // the forward walk's stream: the rhs goes into the multipliers' stream
-    Real* L = sp ? nullptr : (factor_walk_mode<Real>(b) == kFactorStoreL ? static_cast<Real*>(b->Lm) : nullptr);
+    Real* L = factor_walk_mode<Real>(b) == kFactorStoreL ? static_cast<Real*>(b->Lm) : nullptr;
     for (int k = 0; k < b->ir_steps; ++k) {
         IrArgs<Real> a{sp ? P->d_k1_bus_s : P->d_k1_bus, sp ? P->d_k1_ent_s : P->d_k1_ent, nr.k1_nbus, P->d_Y,
                        row_edits(b), b->V, b->S, b->mask, P->d_colmap, L ? L : A, X, Xs, b->tile_active, nr.n, nr.nY,
@@ -962,9 +984,9 @@ void refine_fp64(g2g_batch_s* b, double eps, int T)
         else k_ir_residual<Real, false><<<T * splits, kLanes * kMismatchWaves, 0, b->stream>>>(a);
         HIPCHK(hipGetLastError());
         if (sp) {
-            launch_factor_split<Real>(P, A, static_cast<Real*>(b->U), b->a_stride, b->u_stride, b->tile_active,
-                                      b->jmax, b->clamped, b->error, b->active_rows, T, eps,
-                                      static_cast<Real*>(b->pend), b->stream);
+            launch_factor_split<Real>(P, L ? L : A, static_cast<Real*>(b->U), b->a_stride, b->u_stride,
+                                      b->tile_active, b->jmax, b->clamped, b->error, b->active_rows, T, eps,
+                                      static_cast<Real*>(b->pend), b->stream, L ? kForwardOnly : kFactorFull);
             launch_backward_split<Real>(P, static_cast<const Real*>(b->U), b->u_stride, b->tile_active, X,
                                         b->error, b->active_rows, T, b->stream);
         } else {
@@ -1791,7 +1813,8 @@ int nr_loop_body(g2g_batch_s* b, int max_iter, double tol, int freeze, double gr
         if (b->split_layout)
             launch_factor_split<Real>(b->plan, static_cast<const Real*>(b->A), static_cast<Real*>(b->U), b->a_stride,
                                       b->u_stride, b->tile_active, b->jmax, b->clamped, b->error, b->active_rows,
-                                      split_tiles(b), eps, static_cast<Real*>(b->pend), b->stream);
+                                      split_tiles(b), eps, static_cast<Real*>(b->pend), b->stream,
+                                      factor_walk_mode<Real>(b), multiplier_stream<Real>(b));
         else
             launch_factor<Real>(b->plan, static_cast<const Real*>(b->A), static_cast<Real*>(b->U), b->a_stride,
                                 b->u_stride, b->tile_active, b->jmax, b->clamped, b->error, b->active_rows, b->T,

@@ -1160,7 +1160,6 @@ template <typename Real, int W, bool SPLIT, int RG, int MODE>
 __global__ __launch_bounds__((kLanes * factor_waves<W, SPLIT, MODE>())) void k_factor(FactorArgs<Real> a)
 {
     static_assert(!SPLIT || W == 1, "a split-walk workgroup has one walker");
-    static_assert(!SPLIT || MODE == kFactorFull, "the split walk factorizes in full");
     constexpr int RW = SPLIT ? kSplitRingF : RG > 0 ? RG : W;  // ring geometry (RG: another walker count's)
     constexpr int kCh = value_chunk(sizeof(Real), RW), kNch = value_ring_slots(sizeof(Real), RW);
     static_assert((kNch - 2) * kCh >= 6 + 4 * kFastC2 - 1, "the ring window spans a two-column step's values");
@@ -2470,6 +2469,8 @@ template __global__ void k_factor<float, 2, false, 0, kFactorFull>(FactorArgs<fl
 template __global__ void k_factor<float, 2, false, kHalfRingGeometry, kFactorFull>(FactorArgs<float>);
 template __global__ void k_factor<double, 1, true, 0, kFactorFull>(FactorArgs<double>);
 template __global__ void k_factor<float, 1, true, 0, kFactorFull>(FactorArgs<float>);
+template __global__ void k_factor<float, 1, true, 0, kFactorStoreL>(FactorArgs<float>);
+template __global__ void k_factor<float, 1, true, 0, kForwardOnly>(FactorArgs<float>);
 template __global__ void k_factor<float, 1, false, 0, kFactorStoreL>(FactorArgs<float>);
 template __global__ void k_factor<float, 2, false, 0, kFactorStoreL>(FactorArgs<float>);
 template __global__ void k_factor<float, 2, false, kHalfRingGeometry, kFactorStoreL>(FactorArgs<float>);

@@ -137,7 +137,10 @@ constexpr int kHalfRingGeometry = 4;
 // split walk: sets per tile (from kSplitMinD unknowns up), the walker
 // workgroup's value producers, and its ring geometry (as for RW walkers): the
 // factorization's full chunks, whose window spans a two-column step's 30
-// values; the backward substitution's half chunks (a record spans at most 17)
+// values; the backward substitution's half chunks (a record spans at most 17).
+// Two producers in every mode: with a ring of four slots, more only wait
+// (forward-only refinement of 4,001 rows of 6,500 buses: 25.8 ms a solve with
+// two, 28.5 with four, 27.9 with six).
 constexpr int kSplitSets = 32;
 constexpr int kSplitMinD = 2000;
 constexpr int kSplitProducers = 2;

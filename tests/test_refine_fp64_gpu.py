@@ -90,7 +90,7 @@ def test_forward_walk_refinement_equals_a_second_factorization(monkeypatch, grid
     stream; a second full factorization (G2G_IR_REFACTOR=1) gives bitwise the
     same solves.  The 2,000-bus plan has two walkers and columns longer than
     the kernels' unrolled cases; the 118-bus plan one walker.  (The split walk,
-    which a batch of a few tiles would take, refactorizes.)"""
+    which a batch of a few tiles would take, has a test of its own.)"""
     g = syn.grid_c1() if grid == "c1" else syn.grid_118()
     rows = 192
     _say(f"forward-walk refinement {grid} ir={ir}")
@@ -114,3 +114,28 @@ def test_forward_walk_refinement_equals_a_second_factorization(monkeypatch, grid
     assert (st0 == 0).sum() > rows // 2
     np.testing.assert_array_equal(V0, V1)
     np.testing.assert_array_equal(r0, r1)
+
+
+@pytest.mark.parametrize("grid,rows,ir", [("c1", 64, 1), ("c1", 130, 2), ("c2", 65, 1)])
+def test_split_forward_walk_refinement_equals_a_second_factorization(monkeypatch, grid, rows, ir):
+    """The same of the split walk: its programs walk forward only, level by
+    level, over the multipliers stored in its own layout, and hand on pending
+    right-hand sides (pending matrix values stay zero), bitwise the answer of
+    a second split factorization."""
+    g = syn.grid_c1() if grid == "c1" else syn.grid_c2()
+    _say(f"split forward-walk refinement {grid} rows={rows} ir={ir}")
+    p, q = syn.injection_scenarios(g, rows, seed=37)
+    S = (p + 1j * q) / g.sn_mva
+    outs = syn.random_outages(g, rows, seed=38)
+    plan = _capi.Plan.from_grid(g.Ybus, g.pv, g.pq, g.slack)
+    assert plan.info()["n_split"] > 0
+    monkeypatch.setenv("G2G_SPLIT", "1")
+    got = {}
+    for refactor in ("0", "1"):
+        monkeypatch.setenv("G2G_IR_REFACTOR", refactor)
+        B = _batch(plan, S, g.flat_start(), _capi.MIXED, ir, True, outs, g)
+        B.solve(max_iter=10, tol=1e-8)
+        got[refactor] = (B.get_v(), *B.results())
+    for a, b in zip(got["0"], got["1"]):
+        np.testing.assert_array_equal(a, b)
+    assert (got["0"][1] == 0).sum() > rows // 2
