@@ -196,7 +196,7 @@ struct Ring {
         // the next windows need.  (A read and a wait per slot, one after the
         // other, stood on the walk's chain about once in six records.  6,500
         // buses, a factorization of 16,384 rows: FP64, eight slots, 7.04 ms,
-        // now 6.60; FP32, four slots, 3.04, now 2.97.)
+        // 6.60 so; FP32, four slots, 3.04 and 2.97.)
         __device__ __forceinline__ void wait_for(int cl)
         {
             if (failed) return;
