@@ -1259,6 +1259,8 @@ public:
         ensure(dEx_, bytes);
         flow_rows_ = rows;
         flow_m_ = m;
+        flow_live_.assign(static_cast<size_t>(rows), 0);
+        for (int r : live) flow_live_[r] = 1;
         if (live.empty()) return;
         const int cap = std::min<int>(std::max(1, batch_size_), static_cast<int>(live.size()));
         if (!batch_ || batch_->rows < cap) {
@@ -1331,14 +1333,14 @@ protected:
             hipchk(hipMemcpy(p, d->p, static_cast<size_t>(flow_rows_) * m * sizeof(double), hipMemcpyDeviceToHost),
                    "hipMemcpy D2H");
         for (int r = 0; r < flow_rows_; ++r)
-            if (res_.status[r] == static_cast<int32_t>(RowStatus::NotSimulated))
-                std::fill_n(p + static_cast<size_t>(r) * m, m, std::nan(""));
+            if (!flow_live_[r]) std::fill_n(p + static_cast<size_t>(r) * m, m, std::nan(""));
         return a;
     }
     Branches br_;
     std::vector<std::vector<int>> trips_;  // tripped branches per row
     DevBufPtr dOr_, dEx_;                  // branch currents, rows x m
     int flow_rows_ = 0, flow_m_ = 0;
+    std::vector<char> flow_live_;          // the rows they were computed for (res_ may be a later run's)
     bool flows_ = false;
 
     std::unique_ptr<Grid> grid_;

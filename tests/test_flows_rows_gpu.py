@@ -53,3 +53,27 @@ def test_flows_match_the_closed_form(n, m, rows):
         assert _capi.lib().g2g_batch_branch_flows(B._h, m, P(f), P(t), P(y4), P(bo), P(be), P(tp), P(bad),
                                                   ctypes.c_void_p(do.data_ptr()),
                                                   ctypes.c_void_p(de.data_ptr())) == _capi.G2G_ERR_INVALID
+
+
+@pytest.mark.parametrize("rows_then", [40, 3])
+def test_flows_outlive_a_run_that_fails(rows_then):
+    """The currents of one run stay readable, as they were computed, after a later
+    run (of as many rows or of fewer) that raised before it solved anything."""
+    from gpusim2grid_amd.facades import InjectionSweepGPU
+    from gpusim2grid_amd.warmstart import WarmStart
+    g, other = syn.grid_118(), syn.grid_c0()
+    f = InjectionSweepGPU((g.Ybus, g.flat_start(), g.Sbus, np.array([g.slack]), np.array([1.0]), g.pv, g.pq),
+                          init_from_n_powerflow=False, nb_iter=8)
+    f.set_branch_data(*g.branch_data(), bus_vn_kv=np.full(g.n_bus, 225.0), sn_mva=g.sn_mva)
+    p, q = syn.injection_scenarios(g, 40, seed=51)
+    f.set_injections(p, q, g.sn_mva)
+    f.compute(batch_size=16)
+    f.compute_flows()
+    orr, ex = f.or_amps, f.ex_amps
+    assert np.isfinite(orr).all() and orr.shape == (40, g.n_branch)
+    f.set_injections(p[:rows_then], q[:rows_then], g.sn_mva)
+    f.set_warm_start(WarmStart(other.n_bus, other.pv, other.pq, other.slack, np.abs(other.flat_start()), n_hidden=16))
+    with pytest.raises(Exception, match="MLP"):  # another grid's network
+        f.compute(batch_size=16)
+    np.testing.assert_array_equal(f.or_amps, orr)
+    np.testing.assert_array_equal(f.ex_amps, ex)
