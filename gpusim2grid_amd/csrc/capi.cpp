@@ -343,6 +343,12 @@ struct g2g_plan_s {
 
 constexpr size_t kPinnedUpload = 128 << 10;  // bytes of a pinned upload half
 
+// the row solver's counters: {Newton updates (64 bits), largest iteration,
+// list length, rows left, -, clocks of three phases (64 bits each)}
+constexpr int kRowCnt = 12, kRowClocks = 6;
+// ints of a batch's h_active
+constexpr int kHostRow = 4, kHostError = 20, kHostRequeued = 21, kHostInts = 32;
+
 // staging buffers of the streamed-row calls
 enum StageBuf { kStSlots, kStS, kStV, kStEdPtr, kStEdEnt, kStEdDelta, kStMask, kStSg, kStVg, kStageBufs };
 
@@ -382,8 +388,9 @@ struct g2g_batch_s {
     int* clamped = nullptr;
     int* error = nullptr;     // stream kernels' give-up flag
     // one pinned allocation: h_active {rows and tiles still iterating, rows
-    // restarted; [4..8] row_cnt; [9] error}, the staging halves of small Sbus /
-    // V uploads, and the results (status, iterations, residuals) of rows_pad rows
+    // restarted; kHostRow: row_cnt; kHostError; kHostRequeued}, the staging
+    // halves of small Sbus / V uploads, and the results (status, iterations,
+    // residuals) of rows_pad rows
     int* h_active = nullptr;
     unsigned char* h_up[2] = {nullptr, nullptr};
     bool up_pending[2] = {false, false};  // a staged upload may still be read
@@ -474,7 +481,7 @@ struct g2g_batch_s {
     void* stage[kStageBufs] = {};
     size_t stage_cap[kStageBufs] = {};
     // row solver: per-workgroup scratch (grown on use), the active rows' list,
-    // and its counters {Newton updates (64 bits), largest iteration, list length, rows left}
+    // and its counters
     unsigned char* row_scratch = nullptr;
     size_t row_scratch_cap = 0;
     int* row_list = nullptr;
@@ -1216,7 +1223,7 @@ void sync_stream(g2g_batch_s* b)
 // queued for the host behind its work
 void queue_solve_read(g2g_batch_s* b, bool statuses)
 {
-    HIPCHK(hipMemcpyAsync(b->h_active + 9, b->error, sizeof(int), hipMemcpyDeviceToHost, b->stream));
+    HIPCHK(hipMemcpyAsync(b->h_active + kHostError, b->error, sizeof(int), hipMemcpyDeviceToHost, b->stream));
     if (statuses && b->active_rows > 0)
         HIPCHK(hipMemcpyAsync(b->h_status, b->status, static_cast<size_t>(b->active_rows) * sizeof(int),
                               hipMemcpyDeviceToHost, b->stream));
@@ -1229,6 +1236,25 @@ struct SolveTimer {
     std::vector<std::pair<int, int>> ph[4];  // mismatch, factor, backward + update, warm start
     std::vector<char> factor_main;          // per factorization: a main-layout walk (not the split walk)
     long long rows_main = 0;                // rows of the main-layout factorizations
+    // row solver launches: all phases in one.  Their shares of its time: the
+    // phases' clocks of some first steps, each phase as often as it ran (a row
+    // has one more mismatch than updates).  And the updates of its slowest row.
+    struct RowPart {
+        int e0, e1;
+        double share[3];
+    };
+    std::vector<RowPart> rows;
+    mutable std::vector<double> rows_ms;  // their times, once read
+    int row_updates = 0;
+    void add_rows(int e0, int e1, const unsigned long long* clk, int R, unsigned long long updates, int slowest)
+    {
+        const double u = static_cast<double>(updates);
+        double w[3] = {clk[0] * (u + R), clk[1] * u, clk[2] * u};
+        if (!(w[0] + w[1] + w[2] > 0.0)) w[updates ? 1 : 0] = 1.0;  // (no whole step was timed)
+        const double sum = w[0] + w[1] + w[2];
+        rows.push_back({e0, e1, {w[0] / sum, w[1] / sum, w[2] / sum}});
+        row_updates = std::max(row_updates, slowest);
+    }
     explicit SolveTimer(g2g_batch_s* bb, int max_launches) : b(bb)
     {
         while (static_cast<int>(b->ev.size()) < 2 * max_launches + 4) {
@@ -1252,8 +1278,18 @@ struct SolveTimer {
             HIPCHK(hipEventElapsedTime(&m, b->ev[ph[k][q].first], b->ev[ph[k][q].second]));
             t += m;
         }
+        for (size_t q = 0; q < rows.size() && k < 3 && !main_only; ++q) {
+            if (q >= rows_ms.size()) {
+                float m = 0.f;
+                HIPCHK(hipEventElapsedTime(&m, b->ev[rows[q].e0], b->ev[rows[q].e1]));
+                rows_ms.push_back(m);
+            }
+            t += rows_ms[q] * rows[q].share[k];
+        }
         return t;
     }
+    // one per Newton update of the slowest row, whichever kernels ran it
+    int factorizations() const { return std::max(static_cast<int>(ph[1].size()), row_updates); }
 };
 
 // Tail compaction.  The LU walk of a tile costs the same whatever number of
@@ -1571,16 +1607,23 @@ bool use_rows(const g2g_batch_s* b, int active_rows)
     return active_rows <= b->n_cu * per_cu;
 }
 
-template <typename Real, bool BL, bool VL>
+template <typename Real, bool BL, bool VL, bool TIMED>
 void launch_row_kernel(const RowShape& s, const RowArgs<Real>& a, int grid, hipStream_t st)
 {
-    HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_row_solve<Real, BL, VL>),
+    HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_row_solve<Real, BL, VL, TIMED>),
                                hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(s.lds)));
-    k_row_solve<Real, BL, VL><<<grid, s.threads, s.lds, st>>>(a);
+    k_row_solve<Real, BL, VL, TIMED><<<grid, s.threads, s.lds, st>>>(a);
     HIPCHK(hipGetLastError());
 }
 
-constexpr int kRowCnt = 5;
+template <typename Real, bool TIMED>
+void launch_row_shape(const RowShape& s, const RowArgs<Real>& a, int grid, hipStream_t st)
+{
+    if (s.blk_lds && s.v_lds) launch_row_kernel<Real, true, true, TIMED>(s, a, grid, st);
+    else if (s.blk_lds) launch_row_kernel<Real, true, false, TIMED>(s, a, grid, st);
+    else if (s.v_lds) launch_row_kernel<Real, false, true, TIMED>(s, a, grid, st);
+    else launch_row_kernel<Real, false, false, TIMED>(s, a, grid, st);
+}
 
 // the buffers of a launch over up to R rows
 template <typename Real>
@@ -1682,10 +1725,9 @@ void launch_rows(g2g_batch_s* b, int R, bool listed, int it, bool decided, int m
     a.updates = reinterpret_cast<unsigned long long*>(b->row_cnt);
     a.last_iter = b->row_cnt + 2;
     a.left = b->row_cnt + 4;
-    if (s.blk_lds && s.v_lds) launch_row_kernel<Real, true, true>(s, a, grid, st);
-    else if (s.blk_lds) launch_row_kernel<Real, true, false>(s, a, grid, st);
-    else if (s.v_lds) launch_row_kernel<Real, false, true>(s, a, grid, st);
-    else launch_row_kernel<Real, false, false>(s, a, grid, st);
+    a.clocks = reinterpret_cast<unsigned long long*>(b->row_cnt + kRowClocks);
+    if (clock) launch_row_shape<Real, false>(s, a, grid, st);
+    else launch_row_shape<Real, true>(s, a, grid, st);
 }
 
 // Runs the R active rows from iteration `it` to their end; last_iter: the
@@ -1703,17 +1745,18 @@ int solve_rows(g2g_batch_s* b, int R, int it, bool decided, int max_iter, double
     const bool listed = R < b->active_rows;
     if (listed && !b->row_list) b->row_list = dalloc<int>(static_cast<size_t>(b->rows_pad));
     launch_rows<Real>(b, R, listed, it, decided, max_iter, tol, freeze, growth, nullptr, 0);
-    tm.ph[1].push_back({e0, tm.mark()});
-    tm.factor_main.push_back(0);
-    HIPCHK(hipMemcpyAsync(b->h_active + 4, b->row_cnt, kRowCnt * sizeof(int), hipMemcpyDeviceToHost, st));
+    const int e1 = tm.mark();
+    HIPCHK(hipMemcpyAsync(b->h_active + kHostRow, b->row_cnt, kRowCnt * sizeof(int), hipMemcpyDeviceToHost, st));
     const bool whole = b->compact_R == 0 && !b->mask;  // the statuses are the batch's final ones if no row is left
     if (whole) queue_solve_read(b, true);
     sync_stream(b);
-    unsigned long long upd = 0;
-    std::memcpy(&upd, b->h_active + 4, sizeof(upd));
+    unsigned long long upd = 0, clk[3];
+    std::memcpy(&upd, b->h_active + kHostRow, sizeof(upd));
+    std::memcpy(clk, b->h_active + kHostRow + kRowClocks, sizeof(clk));
     rows_factored += static_cast<long long>(upd);
-    last_iter = std::max(last_iter, b->h_active[6]);
-    const int left = b->h_active[8];
+    last_iter = std::max(last_iter, b->h_active[kHostRow + 2]);
+    tm.add_rows(e0, e1, clk, R, upd, last_iter);
+    const int left = b->h_active[kHostRow + 4];
     b->solve_read = whole && left == 0;
     if (left > 0) {
         k_count_tiles<<<b->T, kLanes, 0, st>>>(b->status, b->rows_pad, b->tile_active);
@@ -1994,7 +2037,7 @@ void check_stream_error(g2g_batch_s* b, bool statuses = false, bool read = false
         queue_solve_read(b, statuses);
         sync_stream(b);
     }
-    if (b->h_active[9]) throw std::runtime_error("a stream wavefront gave up waiting for its data (results invalid)");
+    if (b->h_active[kHostError]) throw std::runtime_error("a stream wavefront gave up waiting for its data (results invalid)");
 }
 
 void fill_stats(g2g_batch_s* b, const SolveTimer& tm, int e_begin, int e_end, int iterations,
@@ -2014,7 +2057,7 @@ void fill_stats(g2g_batch_s* b, const SolveTimer& tm, int e_begin, int e_end, in
     stats->bytes_factor = static_cast<int64_t>(s.a_len + s.u_len) * static_cast<int64_t>(b->real_size()) *
                           static_cast<int64_t>(b->active_rows);
     stats->rows_factored = rows_factored;
-    stats->n_factor_launches = static_cast<int32_t>(tm.ph[1].size());
+    stats->n_factor_launches = static_cast<int32_t>(tm.factorizations());
     stats->ms_factor_main = tm.ms(1, true);
     stats->rows_factored_main = tm.rows_main;
     for (char m : tm.factor_main) stats->n_factor_main += m ? 1 : 0;
@@ -2129,9 +2172,9 @@ void solve_warm_impl(g2g_batch_s* b, g2g_mlp_s* mlp, const unsigned char* mask, 
     b->restart_on = false;
     mask_islanded_v(b);
     const int e_end = tm.mark();
-    HIPCHK(hipMemcpyAsync(b->h_active + 10, b->requeued, sizeof(int), hipMemcpyDeviceToHost, s));
+    HIPCHK(hipMemcpyAsync(b->h_active + kHostRequeued, b->requeued, sizeof(int), hipMemcpyDeviceToHost, s));
     check_stream_error(b, true);
-    const int R = b->h_active[10];
+    const int R = b->h_active[kHostRequeued];
     fill_stats(b, tm, e_begin, e_end, it, rows_factored, stats);
     if (stats) stats->n_requeued = R;
 }
@@ -2698,9 +2741,9 @@ int g2g_batch_create(g2g_plan_t P, int32_t rows, int32_t precision, int32_t per_
         HIPCHK(hipMemsetAsync(b->error, 0, sizeof(int), b->stream));
         {
             unsigned char* h = nullptr;
-            HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&h), 64 + 2 * kPinnedUpload + rp * 16, hipHostMallocDefault));
+            HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&h), kHostInts * sizeof(int) + 2 * kPinnedUpload + rp * 16, hipHostMallocDefault));
             b->h_active = reinterpret_cast<int*>(h);
-            b->h_up[0] = h + 64;
+            b->h_up[0] = h + kHostInts * sizeof(int);
             b->h_up[1] = b->h_up[0] + kPinnedUpload;
             b->h_res = reinterpret_cast<double*>(b->h_up[1] + kPinnedUpload);
             b->h_status = reinterpret_cast<int*>(b->h_res + rp);

@@ -107,8 +107,8 @@ __global__ void k_collect_rows(const int* status, int rows, int* list, int* n)
 
 // BL: every block in LDS; else the blocks below blk_lds0 (the lowest levels,
 // where most blocks and the least dependence are) are in the workgroup's
-// scratch.  VL: V in LDS, else in the scratch.
-template <typename Real, bool BL, bool VL>
+// scratch.  VL: V in LDS, else in the scratch.  TIMED: with the phases' clocks.
+template <typename Real, bool BL, bool VL, bool TIMED>
 __global__ __launch_bounds__(kRowMaxThreads) void k_row_solve(RowArgs<Real> a)
 {
     using B4 = typename V4<Real>::T;
@@ -197,6 +197,21 @@ __global__ __launch_bounds__(kRowMaxThreads) void k_row_solve(RowArgs<Real> a)
         return __builtin_amdgcn_readfirstlane(s);
     };
 
+    // where the time goes: the clocks of the phases of the workgroup's first
+    // Newton step, in LDS (the solve's time is split in their proportion);
+    // `ends` stops at this moment and `begins` starts.  A build of its own: the
+    // clock reads cost a sweep 1 to 1.5 % (118 buses FP64, 16,384 rows; 2,000
+    // mixed, 777).
+    unsigned long long* const clk = red + 5;
+    auto lap = [&](bool now, int ends, int begins) {
+        if constexpr (TIMED) {
+            if (!now || tid != 0) return;
+            const unsigned long long t = __builtin_readcyclecounter();
+            if (ends >= 0) clk[ends] += t;
+            if (begins >= 0) clk[begins] -= t;
+        }
+    };
+    if (TIMED && tid < 3) clk[tid] = 0ull;
     const int todo = a.list ? *a.list_n : a.rows;
     for (int i = blockIdx.x; i < todo; i += gridDim.x) {
         int row = i;
@@ -414,6 +429,8 @@ __global__ __launch_bounds__(kRowMaxThreads) void k_row_solve(RowArgs<Real> a)
         };
 
         for (;;) {
+            const bool timed = TIMED && i == static_cast<int>(blockIdx.x) && n_upd == 0 && !restarted;
+            lap(timed, -1, 0);
             // F and J at V
             double rmax = 0.0, jmax = 0.0;
             for (int q = tid; q < a.n_fill; q += nt) store(a.fill[q], B4{Real(0), Real(0), Real(0), Real(0)});
@@ -519,6 +536,7 @@ __global__ __launch_bounds__(kRowMaxThreads) void k_row_solve(RowArgs<Real> a)
                 __syncthreads();
                 continue;
             }
+            lap(timed, 0, 1);
             if (st != kActive || it >= a.max_iter) break;
             growth = a.growth;
             decide = true;
@@ -529,6 +547,7 @@ __global__ __launch_bounds__(kRowMaxThreads) void k_row_solve(RowArgs<Real> a)
             }
             sync(lev_lds == 0);
             eliminate(eps, true);
+            lap(timed, 1, 2);
             substitute();
             for (int ir = 0; ir < a.ir_steps; ++ir) {
                 // r = F(V) - J(V) dx in FP64, dV_j = V_j (dVm_j / |V_j| + j dtheta_j); then J d = r
@@ -586,6 +605,7 @@ __global__ __launch_bounds__(kRowMaxThreads) void k_row_solve(RowArgs<Real> a)
             ++iter;
             ++n_upd;
             __syncthreads();
+            lap(timed, 2, -1);
             if (a.max_upd > 0 && n_upd >= a.max_upd) break;  // st: still active
         }
         if (!a.clock && st != kConverged && !(prev < kRowKeep)) {
@@ -609,15 +629,28 @@ __global__ __launch_bounds__(kRowMaxThreads) void k_row_solve(RowArgs<Real> a)
             atomicMax(a.last_iter, iter);
         }
     }
+    if constexpr (TIMED) {
+        // (a first row that made no update, or restarted, leaves no whole step)
+        __syncthreads();
+        if (tid < 3 && static_cast<long long>(clk[2]) > 0) atomicAdd(a.clocks + tid, clk[tid]);
+    }
 }
 
-template __global__ void k_row_solve<float, true, true>(RowArgs<float>);
-template __global__ void k_row_solve<float, true, false>(RowArgs<float>);
-template __global__ void k_row_solve<float, false, true>(RowArgs<float>);
-template __global__ void k_row_solve<float, false, false>(RowArgs<float>);
-template __global__ void k_row_solve<double, true, true>(RowArgs<double>);
-template __global__ void k_row_solve<double, true, false>(RowArgs<double>);
-template __global__ void k_row_solve<double, false, true>(RowArgs<double>);
-template __global__ void k_row_solve<double, false, false>(RowArgs<double>);
+template __global__ void k_row_solve<float, true, true, false>(RowArgs<float>);
+template __global__ void k_row_solve<float, true, false, false>(RowArgs<float>);
+template __global__ void k_row_solve<float, false, true, false>(RowArgs<float>);
+template __global__ void k_row_solve<float, false, false, false>(RowArgs<float>);
+template __global__ void k_row_solve<float, true, true, true>(RowArgs<float>);
+template __global__ void k_row_solve<float, true, false, true>(RowArgs<float>);
+template __global__ void k_row_solve<float, false, true, true>(RowArgs<float>);
+template __global__ void k_row_solve<float, false, false, true>(RowArgs<float>);
+template __global__ void k_row_solve<double, true, true, false>(RowArgs<double>);
+template __global__ void k_row_solve<double, true, false, false>(RowArgs<double>);
+template __global__ void k_row_solve<double, false, true, false>(RowArgs<double>);
+template __global__ void k_row_solve<double, false, false, false>(RowArgs<double>);
+template __global__ void k_row_solve<double, true, true, true>(RowArgs<double>);
+template __global__ void k_row_solve<double, true, false, true>(RowArgs<double>);
+template __global__ void k_row_solve<double, false, true, true>(RowArgs<double>);
+template __global__ void k_row_solve<double, false, false, true>(RowArgs<double>);
 
 }  // namespace g2g

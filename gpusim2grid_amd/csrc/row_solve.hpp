@@ -9,7 +9,7 @@ namespace g2g {
 
 constexpr int kRowMaxEdits = 64;   // a row's Ybus edits kept in LDS
 constexpr int kRowMaxThreads = 1024;
-constexpr int kRowRedBytes = 4 * 8 + 4;  // the workgroup's maxima (two sets of two) and the next slice
+constexpr int kRowRedBytes = 8 * 8;  // the workgroup's maxima (two sets of two), the next slice, three clocks
 // A row that ends unconverged with a residual above this (or not finite) is
 // left as it came, for the tile kernels to finish: the iterates of a row that
 // does not contract amplify rounding, so its last one is the solver's own, and
@@ -69,6 +69,7 @@ struct RowArgs {
     unsigned long long* updates;  // Newton updates summed over the rows
     int* last_iter;               // the largest iteration count
     int* left;                    // rows left as they came
+    unsigned long long* clocks;   // nullable: [3] clocks of some rows' first step (mismatch, factorization, the rest)
 };
 
 constexpr size_t row_align(size_t v) { return (v + 31) / 32 * 32; }
@@ -93,7 +94,7 @@ size_t row_scratch_bytes(int n, int nb, int blk_global, bool v_lds, bool refine)
     return (s + 255) / 256 * 256;
 }
 
-template <typename Real, bool BL, bool VL>
+template <typename Real, bool BL, bool VL, bool TIMED>
 __global__ void k_row_solve(RowArgs<Real> a);
 __global__ void k_collect_rows(const int* status, int rows, int* list, int* n);
 

@@ -93,7 +93,11 @@ typedef struct {
     double ms_factor;       /* factorization + forward substitution              */
     double ms_backward;     /* backward substitution + V update                  */
     int64_t bytes_factor;   /* A- and U-stream bytes of one factorization launch  */
-    int64_t rows_factored;  /* rows summed over the factorization launches       */
+    int64_t rows_factored;  /* rows summed over the factorizations               */
+    /* factorizations: one per Newton update of the slowest row.  (The row
+     * solver runs a row's whole iteration in one launch; its time is split
+     * over the three phases above in proportion to the clocks of sampled
+     * steps, and it has no part in the main-layout figures below.) */
     int32_t n_factor_launches;
     int32_t n_requeued;     /* warm solves: rows restarted from the caller's V   */
     double ms_warm_start;   /* warm solves: MLP inference                        */
