@@ -2932,11 +2932,14 @@ int g2g_batch_branch_flows(g2g_batch_t b, int32_t m, const int32_t* from, const 
             if (from[l] < -1 || from[l] >= n || to[l] < -1 || to[l] >= n)
                 throw std::invalid_argument("branch bus out of range");
         const int rows = b->active_rows;
-        const int n_trip = trip_ptr && trip_branch ? trip_ptr[rows] : 0;
-        for (int r = 0; n_trip > 0 && r < rows; ++r)
-            if (trip_ptr[r + 1] < trip_ptr[r]) throw std::invalid_argument("trip_ptr is not monotone");
-        for (int q = n_trip > 0 ? trip_ptr[0] : 0; q < n_trip; ++q)
-            if (trip_branch[q] < 0 || trip_branch[q] >= m) throw std::invalid_argument("tripped branch out of range");
+        // the rows' ranges, in any order (one that steps back is empty)
+        int n_trip = 0;
+        for (int r = 0; trip_ptr && trip_branch && r < rows; ++r)
+            for (int q = trip_ptr[r]; q < trip_ptr[r + 1]; ++q) {
+                if (trip_branch[q] < 0 || trip_branch[q] >= m)
+                    throw std::invalid_argument("tripped branch out of range");
+                n_trip = std::max(n_trip, q + 1);
+            }
         if (rows <= 0) return;
         const int T = (rows + kLanes - 1) / kLanes;
         DeviceScratch s;

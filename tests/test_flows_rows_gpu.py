@@ -77,3 +77,32 @@ def test_flows_outlive_a_run_that_fails(rows_then):
         f.compute(batch_size=16)
     np.testing.assert_array_equal(f.or_amps, orr)
     np.testing.assert_array_equal(f.ex_amps, ex)
+
+
+def test_trip_lists_that_step_back_are_empty():
+    """A row whose trip_ptr steps back has no tripped branch (the C call reads
+    ranges, it has never asked for them in order), and entries that no row's
+    range covers are not looked at."""
+    g = syn.grid_c0()
+    rows, m = 4, g.n_branch
+    B = _capi.Batch(_capi.Plan.from_grid(g.Ybus, g.pv, g.pq, g.slack), rows)
+    B.set_v(np.tile(g.flat_start() * np.exp(0.1j * np.arange(g.n_bus)), (rows, 1)))
+    f, t = g.branch_from.astype(np.int32), g.branch_to.astype(np.int32)
+    y4 = np.ascontiguousarray(np.stack([g.yff, g.yft, g.ytf, g.ytt], axis=1), dtype=np.complex128)
+    one = np.ones(m)
+    tp = np.array([1, 4, 2, 3, 1], np.int32)  # rows: [1, 4), none, [2, 3), none
+    tb = np.array([m + 7, 5, 0, 9], np.int32)  # the first entry is no row's
+    P = lambda a: a.ctypes.data_as(ctypes.c_void_p)  # noqa: E731
+
+    def flows(*trips):
+        o, e = np.full((rows, m), -1.0), np.full((rows, m), -1.0)
+        rc = _capi.lib().g2g_batch_branch_flows(B._h, m, P(f), P(t), P(y4), P(one), P(one), *trips, P(o), P(e))
+        assert rc == 0
+        return o, e
+
+    plain, tripped = flows(None, None), flows(P(tp), P(tb))
+    for a, b in zip(plain, tripped):
+        a = a.copy()
+        a[0, [5, 0, 9]] = 0.0
+        a[2, 0] = 0.0
+        np.testing.assert_array_equal(a, b)
