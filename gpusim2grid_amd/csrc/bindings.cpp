@@ -1091,6 +1091,8 @@ public:
     // compute_limit_violations (contingency_analysis/__init__.py:589-735)
     bool compute_limit_violations = false;
     double violation_tol = 1e-6;
+    // currents of up to this many bytes (both ends) stay on the device
+    size_t flow_device_bytes_ = size_t{4} << 30;
     double get_violation_rel_tol() const { return violation_rel_tol_; }
     void set_violation_rel_tol(double v)
     {
@@ -1253,10 +1255,25 @@ public:
         std::vector<int> live;
         for (int r = 0; r < rows; ++r)
             if (res_.status[r] != static_cast<int32_t>(RowStatus::NotSimulated)) live.push_back(r);
-        // rows x m on the device, where they stay until they are asked for
+        // rows x m on the device, where they stay until they are asked for; of
+        // more than flow_device_bytes_ in host memory, chunk by chunk (a screen
+        // of any size needs only a chunk's on the device)
         const size_t bytes = static_cast<size_t>(rows) * m * sizeof(double);
-        ensure(dOr_, bytes);
-        ensure(dEx_, bytes);
+        const bool on_device = 2 * bytes <= flow_device_bytes_;
+        flows_ = false;
+        if (on_device) {
+            std::vector<double>().swap(hOr_);
+            std::vector<double>().swap(hEx_);
+            ensure(dOr_, bytes);
+            ensure(dEx_, bytes);
+        } else {
+            dOr_.reset();
+            dEx_.reset();
+            hOr_.resize(static_cast<size_t>(rows) * m);
+            hEx_.resize(static_cast<size_t>(rows) * m);
+        }
+        auto* const all_or = static_cast<unsigned char*>(on_device ? dOr_->p : hOr_.data());
+        auto* const all_ex = static_cast<unsigned char*>(on_device ? dEx_->p : hEx_.data());
         flow_rows_ = rows;
         flow_m_ = m;
         flow_live_.assign(static_cast<size_t>(rows), 0);
@@ -1268,7 +1285,7 @@ public:
             batch_ = std::make_unique<Batch>(*grid_, cap, precision_, 0);
         }
         const int B = batch_->rows;
-        DevBufPtr o, e;  // a chunk's rows, when they are not consecutive
+        DevBufPtr o, e;  // a chunk's rows on the device, when they are not consecutive
         std::vector<int32_t> tp, tb;
         for (size_t c0 = 0; c0 < live.size(); c0 += B) {
             const int k = static_cast<int>(std::min<size_t>(B, live.size() - c0));
@@ -1287,6 +1304,7 @@ public:
                                       n, rn[1], rn[2], 1));
             const size_t row = static_cast<size_t>(m) * sizeof(double);
             auto at = [&](const DevBufPtr& b, size_t r) { return static_cast<unsigned char*>(b->p) + r * row; };
+            auto as_rows = [](unsigned char* q) { return reinterpret_cast<double*>(q); };
             const bool straight = runs.size() == 1;
             if (!straight) {
                 ensure(o, static_cast<size_t>(B) * row);
@@ -1295,18 +1313,19 @@ public:
             check(g2g_batch_branch_flows(batch_->h, m, br_.f.data(), br_.t.data(),
                                          reinterpret_cast<const double*>(y4.data()), br_.base_or.data(),
                                          br_.base_ex.data(), tp.data(), tb.empty() ? nullptr : tb.data(),
-                                         reinterpret_cast<double*>(straight ? at(dOr_, runs[0][0]) : at(o, 0)),
-                                         reinterpret_cast<double*>(straight ? at(dEx_, runs[0][0]) : at(e, 0))));
+                                         as_rows(straight ? all_or + runs[0][0] * row : at(o, 0)),
+                                         as_rows(straight ? all_ex + runs[0][0] * row : at(e, 0))));
+            const hipMemcpyKind kind = on_device ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;
             for (const auto& rn : runs) {
                 if (straight) break;
-                hipchk(hipMemcpy(at(dOr_, rn[0]), at(o, rn[2]), rn[1] * row, hipMemcpyDeviceToDevice), "hipMemcpy D2D");
-                hipchk(hipMemcpy(at(dEx_, rn[0]), at(e, rn[2]), rn[1] * row, hipMemcpyDeviceToDevice), "hipMemcpy D2D");
+                hipchk(hipMemcpy(all_or + rn[0] * row, at(o, rn[2]), rn[1] * row, kind), "hipMemcpy of currents");
+                hipchk(hipMemcpy(all_ex + rn[0] * row, at(e, rn[2]), rn[1] * row, kind), "hipMemcpy of currents");
             }
         }
         flows_ = true;
     }
-    py::array_t<double> get_or_amps() const { return flows(dOr_); }
-    py::array_t<double> get_ex_amps() const { return flows(dEx_); }
+    py::array_t<double> get_or_amps() const { return flows(dOr_, hOr_); }
+    py::array_t<double> get_ex_amps() const { return flows(dEx_, hEx_); }
 
     CArr v_base() const
     {
@@ -1323,13 +1342,15 @@ protected:
         if (!ran_) throw std::runtime_error("call run() first");
     }
     // a host copy of a flow result; rows not simulated read NaN
-    py::array_t<double> flows(const DevBufPtr& d) const
+    py::array_t<double> flows(const DevBufPtr& d, const std::vector<double>& h) const
     {
         if (!flows_) throw std::runtime_error("call compute_flows() first");
         const size_t m = static_cast<size_t>(flow_m_);
         py::array_t<double> a({static_cast<py::ssize_t>(flow_rows_), static_cast<py::ssize_t>(m)});
         double* p = a.mutable_data();
-        if (flow_rows_ > 0 && m > 0)
+        if (!d)
+            std::copy_n(h.begin(), static_cast<size_t>(flow_rows_) * m, p);
+        else if (flow_rows_ > 0 && m > 0)
             hipchk(hipMemcpy(p, d->p, static_cast<size_t>(flow_rows_) * m * sizeof(double), hipMemcpyDeviceToHost),
                    "hipMemcpy D2H");
         for (int r = 0; r < flow_rows_; ++r)
@@ -1338,7 +1359,8 @@ protected:
     }
     Branches br_;
     std::vector<std::vector<int>> trips_;  // tripped branches per row
-    DevBufPtr dOr_, dEx_;                  // branch currents, rows x m
+    DevBufPtr dOr_, dEx_;                  // branch currents, rows x m, on the device ...
+    std::vector<double> hOr_, hEx_;        // ... or in host memory
     int flow_rows_ = 0, flow_m_ = 0;
     std::vector<char> flow_live_;          // the rows they were computed for (res_ may be a later run's)
     bool flows_ = false;
@@ -1925,6 +1947,7 @@ PYBIND11_MODULE(_gpusim2grid, m)
             .def("get_ext_state", &S::get_ext_state)
             .def_readwrite("compute_limit_violations", &S::compute_limit_violations)
             .def_readwrite("violation_tol", &S::violation_tol)
+            .def_readwrite("_flow_device_bytes", &S::flow_device_bytes_)
             .def_property("violation_rel_tol", &S::get_violation_rel_tol, &S::set_violation_rel_tol)
             .def_property("violation_capacity", &S::get_violation_capacity, &S::set_violation_capacity)
             .def("set_limits", &S::set_limits, py::arg("bus_vmin_kv"), py::arg("bus_vmax_kv"),

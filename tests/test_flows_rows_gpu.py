@@ -106,3 +106,29 @@ def test_trip_lists_that_step_back_are_empty():
         a[0, [5, 0, 9]] = 0.0
         a[2, 0] = 0.0
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("batch", [7, 64])
+def test_flows_in_host_memory_equal_those_on_the_device(batch):
+    """A screen's currents past the bound of what the device keeps: the same, row
+    by row (trips, rows not simulated, chunks whose rows are not consecutive)."""
+    from gpusim2grid_amd.facades import ContingencyAnalysisGPU
+    g = syn.grid_118()
+    f = ContingencyAnalysisGPU((g.Ybus, g.flat_start(), g.Sbus, np.array([g.slack]), np.array([1.0]), g.pv, g.pq),
+                               init_from_n_powerflow=False, nb_iter=10)
+    f.set_branch_data(*g.branch_data(), bus_vn_kv=np.full(g.n_bus, 225.0), sn_mva=g.sn_mva)
+    cand = syn.bridges(g.n_bus, g.branch_from, g.branch_to)  # (a bridge's outage splits the grid: not simulated)
+    assert cand.any() and not cand.all()
+    f.add_contingencies_by_branch_id([[int(b)] for b in range(0, 60)])
+    f.compute(batch_size=batch)
+    f.compute_flows()
+    orr, ex = f.or_amps, f.ex_amps
+    f.solver._flow_device_bytes = 2 * orr.nbytes - 1
+    f.compute_flows()
+    np.testing.assert_array_equal(f.or_amps, orr)
+    np.testing.assert_array_equal(f.ex_amps, ex)
+    skipped = np.isnan(orr).all(axis=1)
+    np.testing.assert_array_equal(skipped, cand[:60])
+    f.solver._flow_device_bytes = 2 * orr.nbytes  # (and back)
+    f.compute_flows()
+    np.testing.assert_array_equal(f.or_amps, orr)
