@@ -394,6 +394,7 @@ struct g2g_batch_s {
     int* h_active = nullptr;
     unsigned char* h_up[2] = {nullptr, nullptr};
     bool up_pending[2] = {false, false};  // a staged upload may still be read
+    bool arrays_out = false;              // the caller holds V's and Sbus's device addresses
     int* h_status = nullptr;
     int* h_iters = nullptr;
     double* h_res = nullptr;
@@ -2185,8 +2186,9 @@ T* stage_buf(g2g_batch_s* b, int i, size_t n);
 // Rows x m complex (row stride ld complex; ld = 0 broadcasts) -> tiled
 // [T][m][64].  Host rows of up to kPinnedUpload bytes (a power flow's or a few)
 // go through the batch's pinned half `up` and its kept device staging: no
-// allocation, and the copy need not be waited for.  Larger ones are staged in
-// memory that is given back.
+// allocation, and the copy is waited for only where the caller could look (it
+// holds the arrays' addresses, and may read them on a stream of its own).
+// Larger ones are staged in memory that is given back.
 void to_tiles(g2g_batch_s* b, int up, const double* src, long long ld, int rows, int m, int row0, int on_device,
               double2* dst)
 {
@@ -2215,6 +2217,8 @@ void to_tiles(g2g_batch_s* b, int up, const double* src, long long ld, int rows,
     if (tmp) {
         HIPCHK(hipStreamSynchronize(st));
         dfree(tmp);
+    } else if (b->arrays_out && b->up_pending[up]) {
+        sync_stream(b);
     }
 }
 
@@ -3517,6 +3521,8 @@ int g2g_batch_device_arrays(g2g_batch_t b, void** V_tiles, void** S_tiles)
     return guarded([&] {
         if (b) b->v_bcast = false;  // V changes (or is handed out)
         if (!b) throw std::invalid_argument("null batch");
+        if (b->up_pending[0] || b->up_pending[1]) sync_stream(b);
+        b->arrays_out = true;
         if (V_tiles) *V_tiles = b->V;
         if (S_tiles) *S_tiles = b->S;
     });

@@ -416,7 +416,9 @@ int g2g_batch_stream_take(g2g_batch_t batch, int32_t n, const int32_t *slots, do
                           int32_t on_device);
 
 /* Device pointer of the batch's tiled Sbus array [ceil(rows/64)][n][64]
- * complex (bench and zero-copy callers fill it directly). */
+ * complex (bench and zero-copy callers fill it directly), and of its V.  From
+ * this call on, host uploads of V and Sbus are in place when they return, for
+ * a reader on any stream. */
 int g2g_batch_device_arrays(g2g_batch_t batch, void **V_tiles, void **S_tiles);
 
 /* ---- Learned warm start (no counterpart in the reference, whose ML models are
