@@ -142,7 +142,7 @@ __global__ __launch_bounds__(kRowMaxThreads) void k_row_solve(RowArgs<Real> a)
         V = reinterpret_cast<double2*>(take(static_cast<size_t>(a.n) * sizeof(double2)));
     } else {
         V = reinterpret_cast<double2*>(sc);
-        sc += static_cast<size_t>(a.n) * sizeof(double2);
+        sc += row_align(static_cast<size_t>(a.n) * sizeof(double2));  // (B4 is 32 bytes in FP64)
     }
     B4* const ML = reinterpret_cast<B4*>(at);  // the LDS blocks
     B4* const MG = reinterpret_cast<B4*>(sc);

@@ -89,7 +89,7 @@ template <typename Real>
 size_t row_scratch_bytes(int n, int nb, int blk_global, bool v_lds, bool refine)
 {
     size_t s = static_cast<size_t>(blk_global) * 4 * sizeof(Real);
-    if (!v_lds) s += static_cast<size_t>(n) * sizeof(double2);
+    if (!v_lds) s += row_align(static_cast<size_t>(n) * sizeof(double2));
     if (refine) s += static_cast<size_t>(nb) * 2 * sizeof(Real);
     return (s + 255) / 256 * 256;
 }

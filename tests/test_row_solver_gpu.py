@@ -59,6 +59,8 @@ ATOL = {_capi.FP64: 1e-10, _capi.MIXED: 1e-7}
     (37, 5000, _capi.FP64), (118, 64, _capi.MIXED), (301, 700, _capi.FP64), (997, 300, _capi.FP64),
     (2000, 1, _capi.MIXED), (2000, 300, _capi.MIXED), (2000, 70, _capi.FP64), (2000, 600, _capi.FP64),
     (6500, 1, _capi.FP64), (6500, 300, _capi.MIXED),
+    # V and blocks in the scratch, V an odd number of 16-byte values before the 32-byte blocks
+    (3001, 40, _capi.FP64),
     # two workgroups a CU share the LDS (more rows than CUs), with blocks in the scratch
     (601, 257, _capi.FP64), (997, 257, _capi.MIXED), (1501, 513, _capi.FP64), (1501, 513, _capi.MIXED),
 ])
