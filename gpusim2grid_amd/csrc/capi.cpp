@@ -1582,14 +1582,28 @@ bool rows_possible(const g2g_batch_s* b)
            !(b->per_row_y && b->ed_cap > kRowMaxEdits);
 }
 
+// Newton updates that bring the usual start (flat, a plain sweep's injections)
+// below kRowKeep.  With fewer, rows end unconverged above it and the tile
+// kernels solve them again: a solve of 16,384 rows of 997 buses FP64 with three
+// updates 14.9 ms (7.8 on the tile kernels alone), one row of 6,500 with four
+// 4.5 (3.7).  Measured residuals after k updates: 14 and 37 buses k = 2 3e-5;
+// 118 and 301 k = 2 1e-3, k = 3 5e-7; 601 k = 3 8e-5 (just); 997 k = 3 6e-3, k = 4
+// 3e-5; 2,000 k = 3 1e-4, k = 4 7e-10; 4,501 k = 4 2e-5; 6,500 k = 4 2e-3,
+// k = 5 2e-7 (some rows above); 9,001 k = 5 5e-6 (2 % above).
+int row_min_updates(int nb) { return nb <= 50 ? 2 : nb <= 400 ? 3 : nb <= 5000 ? 4 : 6; }
+
+// budget: the updates of the whole solve (streamed rounds, which hand no row
+// back: any)
+constexpr int kAnyBudget = 1 << 30;
 template <typename Real>
-bool use_rows(const g2g_batch_s* b, int active_rows)
+bool use_rows(const g2g_batch_s* b, int active_rows, int budget = kAnyBudget)
 {
     if (active_rows <= 0 || !rows_possible(b)) return false;
     const RowShape s = row_shape<Real>(b, active_rows);
     if (!s.ok) return false;
     const int env = rows_env();
     if (env >= 0) return env == 1;
+    if (budget < row_min_updates(b->plan->rw.r.nb)) return false;
     // Where the two cross over, measured per solve (tile kernels / row solver, ms).
     // Two workgroups a CU or more, at any count: 118 buses FP64 16,384 rows 1.66 / 0.97; 997 mixed
     // 16,384 rows 10.4 / 6.8, 65,536 36.0 / 27.3, FP64 16,384 13.1 / 11.4, 65,536 50.8 / 45.6.
@@ -1780,7 +1794,7 @@ int nr_loop_body(g2g_batch_s* b, int max_iter, double tol, int freeze, double gr
     int restarts = 0;
     int last_row_iter = 0;      // of the rows the row solver finished
     bool rows_tried = false;
-    if (use_rows<Real>(b, b->active_rows)) {
+    if (use_rows<Real>(b, b->active_rows, max_iter)) {
         rows_tried = true;
         if (solve_rows<Real>(b, b->active_rows, 0, false, max_iter, tol, freeze, growth, tm, rows_factored,
                              last_row_iter) == 0)
@@ -1821,7 +1835,7 @@ int nr_loop_body(g2g_batch_s* b, int max_iter, double tol, int freeze, double gr
         if (*b->h_active == 0) break;
         // few rows left: the row solver takes them to their end, from the
         // batch's own layout
-        if (!rows_tried && use_rows<Real>(b, b->h_active[0])) {
+        if (!rows_tried && use_rows<Real>(b, b->h_active[0], max_iter)) {
             rows_tried = true;
             const int left = solve_rows<Real>(b, b->h_active[0], it, true, max_iter, tol, freeze, growth, tm,
                                               rows_factored, last_row_iter);

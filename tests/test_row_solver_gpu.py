@@ -217,3 +217,43 @@ def test_streamed_rounds(n, prec, monkeypatch):
         V = B.stream_take(np.arange(rows))
         ok = st == 0
         assert np.abs(V[ok] - Vt[ok]).max() < ATOL[prec]
+
+
+def _solve_from(g, S, V0, prec, monkeypatch, env, **kw):
+    if env is None:
+        monkeypatch.delenv("G2G_ROWS", raising=False)
+    else:
+        monkeypatch.setenv("G2G_ROWS", env)
+    print(f"row solver rule n={g.n_bus} rows={S.shape[0]} prec={prec} env={env} {kw}", flush=True)
+    P = _capi.Plan.from_grid(g.Ybus, g.pv, g.pq, g.slack)
+    B = _capi.Batch(P, S.shape[0], precision=prec)
+    B.set_sbus(S)
+    B.set_v(V0)
+    B.solve(tol=1e-8, **kw)
+    return (B.get_v(), *B.results())
+
+
+@pytest.mark.parametrize("n,max_iter,tiles", [(118, 0, True), (118, 2, True), (118, 3, False), (601, 3, True),
+                                              (601, 4, False), (2000, 3, True), (2000, 4, False), (6500, 5, True),
+                                              (6500, 6, False)])
+def test_short_budgets_stay_on_the_tile_kernels(n, max_iter, tiles, monkeypatch):
+    """With too few updates for the usual start the row solver would hand every row
+    back unconverged, so the rule leaves such a solve to the tile kernels whatever
+    its start.  Which solver ran shows in the last bits of rows that converge
+    (here from next to their solution)."""
+    g = _grid(n)
+    S = _S(g, 20, 52)
+    V, st, _, _ = _solve_from(g, S, g.flat_start(), _capi.FP64, monkeypatch, "0", max_iter=10)
+    assert (st == 0).all()
+    rng = np.random.default_rng(5)
+    free = np.concatenate([g.pv, g.pq])
+    V0 = V.copy()
+    V0[:, free] *= np.exp(1e-4j * rng.standard_normal((20, free.size)))
+    a = _solve_from(g, S, V0, _capi.FP64, monkeypatch, None, max_iter=max_iter)
+    b = _solve_from(g, S, V0, _capi.FP64, monkeypatch, "0", max_iter=max_iter)
+    np.testing.assert_array_equal(a[1], b[1])
+    np.testing.assert_array_equal(a[2], b[2])
+    if tiles:
+        np.testing.assert_array_equal(a[0], b[0])
+    else:
+        assert (a[1] == 0).all() and 0.0 < np.abs(a[0] - b[0]).max() < ATOL[_capi.FP64]
