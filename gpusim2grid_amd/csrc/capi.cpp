@@ -487,6 +487,10 @@ struct g2g_batch_s {
     size_t row_scratch_cap = 0;
     int* row_list = nullptr;
     int* row_cnt = nullptr;
+    // the clocks of its phases, taken in the batch's first solve (with as many
+    // refinement rounds): each solve's time is split in their proportion
+    int row_clk_ir = -1;
+    double row_clk[3] = {0.0, 0.0, 0.0};
     std::vector<hipEvent_t> ev;
     ~g2g_batch_s()
     {
@@ -1238,8 +1242,8 @@ struct SolveTimer {
     std::vector<char> factor_main;          // per factorization: a main-layout walk (not the split walk)
     long long rows_main = 0;                // rows of the main-layout factorizations
     // row solver launches: all phases in one.  Their shares of its time: the
-    // phases' clocks of some first steps, each phase as often as it ran (a row
-    // has one more mismatch than updates).  And the updates of its slowest row.
+    // phases' clocks (b->row_clk), each phase as often as it ran (a row has one
+    // more mismatch than updates).  And the updates of its slowest row.
     struct RowPart {
         int e0, e1;
         double share[3];
@@ -1247,11 +1251,11 @@ struct SolveTimer {
     std::vector<RowPart> rows;
     mutable std::vector<double> rows_ms;  // their times, once read
     int row_updates = 0;
-    void add_rows(int e0, int e1, const unsigned long long* clk, int R, unsigned long long updates, int slowest)
+    void add_rows(int e0, int e1, int R, unsigned long long updates, int slowest)
     {
         const double u = static_cast<double>(updates);
-        double w[3] = {clk[0] * (u + R), clk[1] * u, clk[2] * u};
-        if (!(w[0] + w[1] + w[2] > 0.0)) w[updates ? 1 : 0] = 1.0;  // (no whole step was timed)
+        double w[3] = {b->row_clk[0] * (u + R), b->row_clk[1] * u, b->row_clk[2] * u};
+        if (!(w[0] + w[1] + w[2] > 0.0)) w[updates ? 1 : 0] = 1.0;  // (no whole step was clocked yet)
         const double sum = w[0] + w[1] + w[2];
         rows.push_back({e0, e1, {w[0] / sum, w[1] / sum, w[2] / sum}});
         row_updates = std::max(row_updates, slowest);
@@ -1741,8 +1745,8 @@ void launch_rows(g2g_batch_s* b, int R, bool listed, int it, bool decided, int m
     a.last_iter = b->row_cnt + 2;
     a.left = b->row_cnt + 4;
     a.clocks = reinterpret_cast<unsigned long long*>(b->row_cnt + kRowClocks);
-    if (clock) launch_row_shape<Real, false>(s, a, grid, st);
-    else launch_row_shape<Real, true>(s, a, grid, st);
+    if (!clock && b->row_clk_ir != b->ir_steps) launch_row_shape<Real, true>(s, a, grid, st);
+    else launch_row_shape<Real, false>(s, a, grid, st);
 }
 
 // Runs the R active rows from iteration `it` to their end; last_iter: the
@@ -1770,7 +1774,11 @@ int solve_rows(g2g_batch_s* b, int R, int it, bool decided, int max_iter, double
     std::memcpy(clk, b->h_active + kHostRow + kRowClocks, sizeof(clk));
     rows_factored += static_cast<long long>(upd);
     last_iter = std::max(last_iter, b->h_active[kHostRow + 2]);
-    tm.add_rows(e0, e1, clk, R, upd, last_iter);
+    if (clk[2] > 0) {
+        for (int q = 0; q < 3; ++q) b->row_clk[q] = static_cast<double>(clk[q]);
+        b->row_clk_ir = b->ir_steps;
+    }
+    tm.add_rows(e0, e1, R, upd, last_iter);
     const int left = b->h_active[kHostRow + 4];
     b->solve_read = whole && left == 0;
     if (left > 0) {

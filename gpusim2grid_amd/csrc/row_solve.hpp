@@ -69,7 +69,7 @@ struct RowArgs {
     unsigned long long* updates;  // Newton updates summed over the rows
     int* last_iter;               // the largest iteration count
     int* left;                    // rows left as they came
-    unsigned long long* clocks;   // nullable: [3] clocks of some rows' first step (mismatch, factorization, the rest)
+    unsigned long long* clocks;   // [3] clocks of some rows' first step: mismatch, factorization, the rest (timed build)
 };
 
 constexpr size_t row_align(size_t v) { return (v + 31) / 32 * 32; }

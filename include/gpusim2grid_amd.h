@@ -96,8 +96,9 @@ typedef struct {
     int64_t rows_factored;  /* rows summed over the factorizations               */
     /* factorizations: one per Newton update of the slowest row.  (The row
      * solver runs a row's whole iteration in one launch; its time is split
-     * over the three phases above in proportion to the clocks of sampled
-     * steps, and it has no part in the main-layout figures below.) */
+     * over the three phases above in proportion to the clocks of some steps of
+     * the batch's first solve, and it has no part in the main-layout figures
+     * below.) */
     int32_t n_factor_launches;
     int32_t n_requeued;     /* warm solves: rows restarted from the caller's V   */
     double ms_warm_start;   /* warm solves: MLP inference                        */

@@ -21,10 +21,12 @@ def _stats(g, S, prec, rows_on, monkeypatch, edits=None, max_iter=10):
     B = _capi.Batch(_capi.Plan.from_grid(g.Ybus, g.pv, g.pq, g.slack), S.shape[0], precision=prec,
                     per_row_ybus=edits is not None)
     B.set_sbus(S)
-    B.set_v(g.flat_start())
     if edits is not None:
         B.set_ybus_edits(*edits)
-    s = B.solve(max_iter=max_iter, tol=1e-8)
+    for _ in range(2):  # (the phases' clocks are the first solve's)
+        B.set_v(g.flat_start())
+        s = B.solve(max_iter=max_iter, tol=1e-8)
+        _check_phases(s)
     return s, B.results()
 
 
@@ -44,8 +46,6 @@ def test_factorizations_and_phases(n, rows, prec, hard, monkeypatch):
     s, (st, it, _) = _stats(g, S, prec, None, monkeypatch)
     t, (stt, itt, _) = _stats(g, S, prec, "0", monkeypatch)
     np.testing.assert_array_equal(st, stt)
-    _check_phases(s)
-    _check_phases(t)
     # one factorization per Newton update of the slowest row
     assert t["n_factor_launches"] == itt.max() and s["n_factor_launches"] == it.max()
     assert s["rows_factored"] == it.sum()
@@ -63,7 +63,6 @@ def test_a_tail_on_the_row_solver_counts_on(monkeypatch):
     t, (stt, itt, _) = _stats(g, S, _capi.FP64, "0", monkeypatch, edits)
     np.testing.assert_array_equal(st, stt)
     np.testing.assert_array_equal(it, itt)
-    _check_phases(s)
     assert s["iterations"] == t["iterations"] and s["n_factor_launches"] == t["n_factor_launches"] == it.max()
 
 
