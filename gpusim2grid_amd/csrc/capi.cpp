@@ -344,7 +344,7 @@ struct g2g_plan_s {
 constexpr size_t kPinnedUpload = 128 << 10;  // bytes of a pinned upload half
 
 // the row solver's counters: {Newton updates (64 bits), largest iteration,
-// list length, rows left, -, clocks of three phases (64 bits each)}
+// list length, rows left (first round, the others), clocks of three phases (64 bits each)}
 constexpr int kRowCnt = 12, kRowClocks = 6;
 // ints of a batch's h_active
 constexpr int kHostRow = 4, kHostError = 20, kHostRequeued = 21, kHostInts = 32;
@@ -1668,6 +1668,18 @@ int row_grid(const g2g_batch_s* b, const RowShape& s, int R)
 
 // The launches over R rows (listed: the active ones among more).  clock
 // (nullable), max_upd: a streamed round's iteration clock and its updates.
+//
+// A batch of more than two rounds of workgroups runs its first round by itself;
+// the launch of the others leaves them all if that round left a row.  The tile
+// kernels solve a row that is left from its start, and cost one row about what
+// they cost the batch, so rows solved here beside it are work on top.  Which
+// rows go where depends on the rows alone.  A solve of ten updates (ms: so /
+// with every row tried here to its budget / tile kernels alone): 118 buses
+// FP64, 16,384 rows, 1 % of them without a solution 3.52 / 4.13 / 3.36; 997 FP64,
+// 16,384, 10 % 24.8 / 37.9 / 24.2, 0.1 % (none in the first round) 28.4 / 28.3 /
+// 20.8; 2,000 mixed, 8,192, all 23.5 / 36.7 / 23.1; one round, 6,500 FP64, 256,
+// 1 % 12.0 / 12.5 / 9.4.  Batches that all converge pay the second launch: 118
+// FP64, 16,384 rows 0.905 -> 0.927 ms of kernel, 2,000 mixed, 777 0.744 -> 0.752.
 template <typename Real>
 void launch_rows(g2g_batch_s* b, int R, bool listed, int it, bool decided, int max_iter, double tol, int freeze,
                  double growth, const int* clock, int max_upd)
@@ -1716,6 +1728,7 @@ void launch_rows(g2g_batch_s* b, int R, bool listed, int it, bool decided, int m
     a.iters = b->iters;
     a.res = b->res;
     a.jmax = b->jmax;
+    a.row0 = 0;
     a.rows = b->active_rows;
     a.list = listed ? b->row_list : nullptr;
     a.list_n = b->row_cnt + 3;
@@ -1728,6 +1741,7 @@ void launch_rows(g2g_batch_s* b, int R, bool listed, int it, bool decided, int m
     a.freeze = freeze;
     a.growth = growth;
     a.contraction = b->contraction;
+    a.look = clock ? 1 << 30 : kRowLook;
     a.pivot_eps = b->precision == G2G_MIXED ? 1e-5 : 1e-12;
     a.ir_steps = b->ir_steps;
     if (b->streaming || b->restart_on) a.it0 = b->it0;
@@ -1745,8 +1759,20 @@ void launch_rows(g2g_batch_s* b, int R, bool listed, int it, bool decided, int m
     a.last_iter = b->row_cnt + 2;
     a.left = b->row_cnt + 4;
     a.clocks = reinterpret_cast<unsigned long long*>(b->row_cnt + kRowClocks);
-    if (!clock && b->row_clk_ir != b->ir_steps) launch_row_shape<Real, true>(s, a, grid, st);
-    else launch_row_shape<Real, false>(s, a, grid, st);
+    const bool timed = !clock && b->row_clk_ir != b->ir_steps;
+    auto launch = [&] {
+        if (timed) launch_row_shape<Real, true>(s, a, grid, st);
+        else launch_row_shape<Real, false>(s, a, grid, st);
+    };
+    const bool first = !clock && !listed && R > 2 * grid;
+    if (first) a.rows = grid;
+    launch();
+    if (!first) return;
+    a.row0 = grid;
+    a.rows = b->active_rows;
+    a.stop = a.left;
+    a.left = b->row_cnt + 5;
+    launch();  // (the same kernel: another's code is not in the instruction caches, 25 us of that batch)
 }
 
 // Runs the R active rows from iteration `it` to their end; last_iter: the
@@ -1779,7 +1805,7 @@ int solve_rows(g2g_batch_s* b, int R, int it, bool decided, int max_iter, double
         b->row_clk_ir = b->ir_steps;
     }
     tm.add_rows(e0, e1, R, upd, last_iter);
-    const int left = b->h_active[kHostRow + 4];
+    const int left = b->h_active[kHostRow + 4] + b->h_active[kHostRow + 5];
     b->solve_read = whole && left == 0;
     if (left > 0) {
         k_count_tiles<<<b->T, kLanes, 0, st>>>(b->status, b->rows_pad, b->tile_active);

@@ -211,16 +211,20 @@ __global__ __launch_bounds__(kRowMaxThreads) void k_row_solve(RowArgs<Real> a)
         }
     };
     if (TIMED && tid < 3) clk[tid] = 0ull;
-    const int todo = a.list ? *a.list_n : a.rows;
+    const int todo = a.list ? *a.list_n : a.rows - a.row0;
+    if (a.stop && *a.stop > 0) {
+        if (blockIdx.x == 0 && tid == 0) atomicAdd(a.left, todo);
+        return;
+    }
     for (int i = blockIdx.x; i < todo; i += gridDim.x) {
-        int row = i;
+        int row = a.row0 + i;
         if (a.list) {
             row = a.list[i];
         } else if (gridDim.x % 64 == 0 && i - static_cast<int>(blockIdx.x) + static_cast<int>(gridDim.x) <= todo) {
             // workgroup g runs on XCD g % 8: rows 8 r .. 8 r + 7, whose V and
             // Sbus share cache lines, go to one XCD's workgroups
             const int g = blockIdx.x, s = g / kXcds;
-            row = i - g + ((s / 8) * kXcds + g % kXcds) * 8 + s % 8;
+            row = a.row0 + i - g + ((s / 8) * kXcds + g % kXcds) * 8 + s % 8;
         }
         if (!a.list && a.status[row] != kActive) continue;
         const size_t tile = static_cast<size_t>(row) / kLanes;
@@ -250,7 +254,7 @@ __global__ __launch_bounds__(kRowMaxThreads) void k_row_solve(RowArgs<Real> a)
         bool decide = !a.skip_first;
         int iter = a.clock ? *a.clock + a.iter0 : a.iter0, st = kActive, n_upd = 0;
         double jm = 0.0;
-        int turn = 0;
+        int turn = 0, look = a.look;  // look: the update from which on a row must contract
         if (tid == 0) {
             *slice_next = n_wave;
             red[0] = red[1] = 0ull;
@@ -518,6 +522,8 @@ __global__ __launch_bounds__(kRowMaxThreads) void k_row_solve(RowArgs<Real> a)
                          r > a.contraction * prev * prev)
                     st = kRejected;
                 else if (it >= budget) st = r < a.tol ? kConverged : (wrow ? kRejected : kMaxIter);
+                // (not a row on a learned start, which has its own rejection rule)
+                else if (it >= look && !wrow && r > kRowContract * prev && r >= kRowKeep) st = kRowGivenUp;
             }
             prev = r;
             if (st == kRejected && wrow) {
@@ -525,6 +531,7 @@ __global__ __launch_bounds__(kRowMaxThreads) void k_row_solve(RowArgs<Real> a)
                 wrow = false;
                 budget = it + a.restart_max_iter;
                 restarted = true;
+                look = it + a.look;
                 for (int q = tid; q < a.n; q += nt) {
                     const int bus = a.bus_of[q];
                     V[q] = a.v0_row ? a.V0[bus] : a.V0[vbase + static_cast<size_t>(bus) * kLanes];

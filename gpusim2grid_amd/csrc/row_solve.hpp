@@ -16,6 +16,14 @@ constexpr int kRowRedBytes = 8 * 8;  // the workgroup's maxima (two sets of two)
 // callers keep getting the one they always got.  (Not in streamed rounds, where
 // a row's V moves on with every launch.)
 constexpr double kRowKeep = 1e-4;
+// Such a row is given up early: from its third update on, when an update does
+// not halve a residual above kRowKeep.  (By the oracle, from the flat start, 14
+// to 6,500 buses, injections scaled up to the last row that converges: every
+// row that converges halves it or better from the third update on, nearly all
+// others fail to by their fourth.)
+constexpr int kRowLook = 3;
+constexpr double kRowContract = 0.5;
+constexpr int kRowGivenUp = 99;  // such a row's status inside the kernel
 
 template <typename Real>
 struct RowArgs {
@@ -44,7 +52,7 @@ struct RowArgs {
     int* iters;
     double* res;
     double* jmax;
-    int rows;
+    int row0, rows;         // rows [row0, rows)
     const int* list;        // nullable: the active rows; count at list_n
     const int* list_n;
     int iter0, skip_first;  // first iteration; 1: its statuses are already decided
@@ -54,6 +62,7 @@ struct RowArgs {
     double tol;
     int freeze;
     double growth, contraction;
+    int look;               // kRowLook (streamed rounds, which hand no row back: never)
     double pivot_eps;
     int ir_steps;           // refinement rounds with the FP64 residual
     // learned starts (null without)
@@ -69,6 +78,7 @@ struct RowArgs {
     unsigned long long* updates;  // Newton updates summed over the rows
     int* last_iter;               // the largest iteration count
     int* left;                    // rows left as they came
+    const int* stop;              // nullable: a launch before this left rows: leave all
     unsigned long long* clocks;   // [3] clocks of some rows' first step: mismatch, factorization, the rest (timed build)
 };
 

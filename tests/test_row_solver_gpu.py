@@ -257,3 +257,27 @@ def test_short_budgets_stay_on_the_tile_kernels(n, max_iter, tiles, monkeypatch)
         np.testing.assert_array_equal(a[0], b[0])
     else:
         assert (a[1] == 0).all() and 0.0 < np.abs(a[0] - b[0]).max() < ATOL[_capi.FP64]
+
+
+@pytest.mark.parametrize("where", [[5], [4990], [5, 4990], list(range(0, 5000, 7))])
+@pytest.mark.parametrize("prec", [_capi.FP64, _capi.MIXED])
+def test_hard_rows_among_many(prec, where, monkeypatch):
+    """Rows with no solution among more rows than two rounds of workgroups: found in
+    the first round they send the rows after it to the tile kernels; found later
+    they alone go there.  Either way every answer is the tile kernels', those of
+    the hard rows and of the rows sent along with them bit for bit."""
+    g = _grid(118)
+    S = _S(g, 5000, 53)
+    S[where] *= 12.0
+    V, st, it, res = _solve_from(g, S, g.flat_start(), prec, monkeypatch, None, max_iter=10)
+    Vt, stt, itt, rest = _solve_from(g, S, g.flat_start(), prec, monkeypatch, "0", max_iter=10)
+    np.testing.assert_array_equal(st, stt)
+    assert (st[where] != 0).all() and (np.delete(st, where) == 0).all()
+    exact = np.arange(4200, 5000) if where[0] < 10 else np.array(where)
+    exact = np.union1d(exact, where)
+    for a, b in ((V, Vt), (it, itt), (res, rest)):
+        np.testing.assert_array_equal(a[exact], b[exact])
+    ok = st == 0
+    assert np.abs(V[ok] - Vt[ok]).max() < ATOL[prec]
+    if prec == _capi.FP64:
+        np.testing.assert_array_equal(it, itt)
