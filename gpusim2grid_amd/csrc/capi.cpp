@@ -1614,15 +1614,21 @@ bool use_rows(const g2g_batch_s* b, int active_rows, int budget = kAnyBudget)
     // One a CU, by what a row keeps in the scratch (in the L2 and last-level cache) beside the LDS:
     //   none but V   2,000 mixed 12,288 rows 10.6 / 9.0, 14,336 11.7 / 10.5, 16,384 12.1 / 11.9
     //   FP64         2,000 (176 KB) 8,192 rows 15.0 / 11.5, 12,288 19.0 / 17.1; 3,000 (346 KB) 4,096 14.1 / 11.4;
-    //                4,500 (598 KB) 2,048 13.0 / 9.6; 6,500 (876 KB) 768 10.1 / 7.6, 1,024 10.7 / 11.0
+    //                4,500 (598 KB) 2,048 13.0 / 9.6; 6,500 (876 KB) 768 10.1 / 7.6, 1,024 10.7 / 11.0;
+    //                9,001 (1,354 KB) 768 15.0 / 13.7 (from 10,240 buses on the LDS does not hold its part)
     //   mixed        3,000 (116 KB) 8,192 14.0 / 13.4; 4,500 (254 KB) 4,096 10.3 / 10.9;
-    //                6,500 (409 KB) 2,048 11.3 / 9.9
+    //                6,500 (409 KB) 2,048 11.3 / 9.9; 9,001 (667 KB) 2,048 19.6 / 18.7;
+    //                10,501 (810 KB) 1,024 14.2 / 12.8, 1,536 20.4 / 19.9, 2,048 23.0 / 26.4;
+    //                13,001 (1,036 KB) 512 10.7 / 8.8, 1,024 16.3 / 17.6; 16,001 (1,312 KB) 512 13.9 / 15.2
+    // With 0 - 2 outages a row, or with FP64-residual refinement, the row solver wins by as much or
+    // more on both sides of these lines: 2,000 mixed 14,336 rows with outages 13.6 / 10.8, 997 FP64
+    // 65,536 53.8 / 47.4; refined 2,000 mixed 12,288 rows 17.5 / 16.4, 6,500 2,048 17.1 / 15.3.
     if (s.per_cu >= 2) return true;
     const size_t kb = s.scratch >> 10;
     int per_cu;  // rows a CU
     if (s.blk_lds) per_cu = 56;
     else if (sizeof(Real) == 8) per_cu = kb <= 200 ? 48 : kb <= 400 ? 16 : kb <= 640 ? 8 : 3;
-    else per_cu = kb <= 200 ? 32 : 8;
+    else per_cu = kb <= 200 ? 32 : kb <= 700 ? 8 : kb <= 850 ? 4 : kb <= 1100 ? 2 : 1;
     return active_rows <= b->n_cu * per_cu;
 }
 

@@ -281,3 +281,16 @@ def test_hard_rows_among_many(prec, where, monkeypatch):
     assert np.abs(V[ok] - Vt[ok]).max() < ATOL[prec]
     if prec == _capi.FP64:
         np.testing.assert_array_equal(it, itt)
+
+
+@pytest.mark.parametrize("n,rows,tiles", [(13001, 512, False), (13001, 513, True)])
+def test_large_grids_change_over_at_few_rows(n, rows, tiles, monkeypatch):
+    """Past the sizes whose blocks the caches hold, mixed precision: two rows a CU on
+    the row solver, more on the tile kernels (which ran shows in the last bits)."""
+    g = _grid(n)
+    S = 0.8 * _S(g, 8, 54)[np.arange(rows) % 8]
+    a = _solve_from(g, S, g.flat_start(), _capi.MIXED, monkeypatch, None, max_iter=10)
+    b = _solve_from(g, S, g.flat_start(), _capi.MIXED, monkeypatch, "0", max_iter=10)
+    assert (a[1] == 0).all() and (b[1] == 0).all()
+    assert np.abs(a[0] - b[0]).max() < ATOL[_capi.MIXED]
+    assert np.array_equal(a[0], b[0]) == tiles
