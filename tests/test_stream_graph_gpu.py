@@ -20,8 +20,9 @@ def _say(msg):
 
 @pytest.mark.parametrize("prec,refine", [(_capi.FP64, False), (_capi.MIXED, False), (_capi.MIXED, True)])
 def test_graph_rounds_equal_eager_rounds(prec, refine):
-    """refine: one FP64-residual refinement round per update, whose
-    multiplier-storing factorization and forward-only walk are captured too."""
+    """refine: one FP64-residual refinement round per update.  (At this size the
+    rounds are the row solver's; test_tile_solver_gpu.py runs them on the tile
+    kernels, multiplier-storing factorization and forward-only walk captured.)"""
     g = syn.grid_118()
     rows, slots = 500, 128
     _say(f"stream graph prec={prec} refine={refine}")
