@@ -902,7 +902,6 @@ struct EditLists {
     }
 };
 
-// room for cap edits per row (the lists kept when keep is set)
 // A captured round holds the buffers' addresses: it goes before one of them
 // is replaced (the next round is captured again).
 void drop_round_graph(g2g_batch_s* b)
@@ -915,6 +914,7 @@ void drop_round_graph(g2g_batch_s* b)
     b->graph = nullptr;
 }
 
+// room for cap edits per row (the lists kept when keep is set)
 void ensure_edit_cap(g2g_batch_s* b, int cap, bool keep)
 {
     if (cap <= b->ed_cap) return;

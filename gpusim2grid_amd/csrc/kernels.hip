@@ -2030,7 +2030,6 @@ __global__ void k_fill_int(int* __restrict__ p, int v, long long n)
     if (gid < n) p[gid] = v;
 }
 
-// tile_active[t] = rows of tile t still iterating
 // a solve's start: rows [0, active) iterate, the others are not simulated
 __global__ void k_init_rows(int active, int rows_pad, int* __restrict__ status, int* __restrict__ iters,
                             int* __restrict__ tile_active)
@@ -2042,6 +2041,7 @@ __global__ void k_init_rows(int active, int rows_pad, int* __restrict__ status, 
     if (r % kLanes == 0) tile_active[r / kLanes] = min(max(active - r, 0), kLanes);
 }
 
+// tile_active[t] = rows of tile t still iterating
 __global__ void k_count_tiles(const int* __restrict__ status, int rows_pad, int* __restrict__ tile_active)
 {
     const int t = blockIdx.x;
@@ -2082,8 +2082,7 @@ __global__ void k_move_vals(const T* __restrict__ src, T* __restrict__ dst, cons
 
 // Branch terminal currents on converged V (acpf_nr_kernels.cu:122-182):
 //   I_or = yff V_f + yft V_t,  I_ex = ytf V_f + ytt V_t,  amps = |I| * base current
-// One thread per (tile, branch, lane); outputs tiled [T][m][64].  A side with
-// bus -1 (no terminal) reports 0.
+// A side with bus -1 (no terminal) reports 0.
 // Rows x m outputs, row-major: a workgroup computes a tile's 64 rows of
 // kFlowBranches branches with a lane per row (the tiled V's coalesced reads)
 // and writes them through LDS with a lane per branch, so the caller's layout

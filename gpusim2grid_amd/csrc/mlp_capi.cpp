@@ -409,8 +409,8 @@ int g2g_mlp_create(int32_t n_in, int32_t n_hidden, int32_t n_out, uint64_t seed,
         HIPCHK(hipMemcpy(p->w, h.data(), o * sizeof(float), hipMemcpyHostToDevice));
         HIPCHK(hipMemset(p->m, 0, o * sizeof(float)));
         HIPCHK(hipMemset(p->v, 0, o * sizeof(float)));
-        // the layers' gradients never write the padding between them, which
-        // the gradient norm and the Adam update read: zero it once
+        // (the padding between the layers' gradients is never written; callers
+        // that take the gradients copy it)
         HIPCHK(hipMemset(p->g, 0, o * sizeof(float)));
         p->refresh_weights(nullptr, nullptr);
         HIPCHK(hipDeviceSynchronize());
