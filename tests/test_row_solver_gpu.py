@@ -294,3 +294,69 @@ def test_large_grids_change_over_at_few_rows(n, rows, tiles, monkeypatch):
     assert (a[1] == 0).all() and (b[1] == 0).all()
     assert np.abs(a[0] - b[0]).max() < ATOL[_capi.MIXED]
     assert np.array_equal(a[0], b[0]) == tiles
+
+
+def _net(n, edges, y=1.0 / (0.01 + 0.1j), drop=(), zeros=()):
+    """Ybus of branches with a little charging; `drop`: entries taken out of the
+    pattern one way only; `zeros`: stored entries of value zero."""
+    import scipy.sparse as sp
+    e = np.asarray(edges)
+    f, t = e[:, 0], e[:, 1]
+    Y = sp.coo_matrix((np.concatenate([np.full(2 * len(e), -y), np.full(2 * len(e), y + 0.01j), np.full(n, 1e-3j)]),
+                       (np.concatenate([f, t, f, t, np.arange(n)]), np.concatenate([t, f, f, t, np.arange(n)]))),
+                      shape=(n, n)).tocsr()
+    Y = Y.tolil()
+    for i, j in drop:
+        Y[i, j] = 0
+    Y = Y.tocsr()
+    Y.eliminate_zeros()
+    if zeros:
+        i, j = np.asarray(zeros).T
+        Y = Y + sp.coo_matrix((np.full(len(i), 1e-300), (i, j)), shape=(n, n)).tocsr()
+        Y.data[np.abs(Y.data) < 1e-200] = 0.0
+    Y.sort_indices()
+    return Y
+
+
+FORMS = {
+    "chain": (300, [(i, i + 1) for i in range(299)], dict(y=1.0 / (1e-4 + 1e-3j))),
+    "star": (90, [(0, i) for i in range(1, 90)], {}),
+    "star past a record's terms": (200, [(0, i) for i in range(1, 200)], {}),
+    "complete": (8, [(i, j) for i in range(8) for j in range(i)], {}),
+    "entries one way only": (60, [(i, (i + 1) % 60) for i in range(60)] + [(i, i + 2) for i in range(0, 58, 2)],
+                             dict(drop=[(3, 4), (10, 12), (58, 59), (0, 2)])),
+    "stored zeros": (60, [(i, (i + 1) % 60) for i in range(60)],
+                     dict(zeros=[(2, 40), (40, 2), (5, 30), (33, 11)])),
+}
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("prec", [_capi.FP64, _capi.MIXED])
+def test_forms_of_the_bus_graph(form, prec, monkeypatch):
+    """Graphs at and past the record format's bounds (which the tile kernels solve;
+    denser ones no plan takes), patterns that are not symmetric, stored zeros, fixed buses off the graph."""
+    n, edges, kw = FORMS[form]
+    Y = _net(n, edges, **kw)
+    rng = np.random.default_rng(8)
+    slack, pv, rest = 1, np.array([0, n // 2]), np.setdiff1d(np.arange(n), [0, 1, n // 2])
+    pq = rest[:-2]  # (the last two buses are fixed)
+    scale = 0.3 / n
+    S = -scale * (rng.uniform(0.5, 1.5, (70, n)) + 0.3j * rng.uniform(0.5, 1.5, (70, n)))
+    V0 = np.ones(n, np.complex128)
+    out = []
+    for env in ("1", "0"):
+        monkeypatch.setenv("G2G_ROWS", env)
+        print(f"form {form} prec={prec} rows_on={env}", flush=True)
+        B = _capi.Batch(_capi.Plan.from_grid(Y, pv, pq, np.array([slack])), 70, precision=prec)
+        B.set_sbus(S)
+        B.set_v(V0)
+        B.solve(max_iter=10, tol=1e-8)
+        out.append((B.get_v(), *B.results()))
+    (V, st, it, _), (Vt, stt, itt, _) = out
+    Vo, sto, ito, _ = orc.nr_batch(Y, V0, S, pv, pq, 10, 1e-8, n_threads=16)
+    assert (sto == 0).all()
+    np.testing.assert_array_equal(st, sto)
+    np.testing.assert_array_equal(stt, sto)
+    assert np.abs(V - Vt).max() < ATOL[prec] and np.abs(V - Vo).max() < ATOL[prec]
+    if prec == _capi.FP64:
+        np.testing.assert_array_equal(it, ito)
