@@ -360,3 +360,42 @@ def test_forms_of_the_bus_graph(form, prec, monkeypatch):
     assert np.abs(V - Vt).max() < ATOL[prec] and np.abs(V - Vo).max() < ATOL[prec]
     if prec == _capi.FP64:
         np.testing.assert_array_equal(it, ito)
+
+
+@pytest.mark.parametrize("where", [[5, 900], [4990]])
+def test_hard_rows_among_learned_starts(where, monkeypatch):
+    """The same from learned starts, some of which fail and restart in the first round
+    before the rest is sent on: statuses, counts and restarts are the tile kernels'."""
+    from gpusim2grid_amd.warmstart import WarmStart
+    g = _grid(118)
+    rows = 5000
+    S = _S(g, rows, 55)
+    S[where] *= 12.0
+    rng = np.random.default_rng(9)
+    ws = WarmStart(g.n_bus, g.pv, g.pq, g.slack, np.abs(g.flat_start()), n_hidden=64, seed=3)
+    mu = np.zeros(ws.n_out, np.float32)
+    mu[1::2] = 1.0
+    ws.mlp.set_normalization(np.zeros(ws.n_in, np.float32), np.ones(ws.n_in, np.float32), mu,
+                             np.full(ws.n_out, 0.6, np.float32))
+    ws.mlp.set_params({k: rng.normal(0, 0.3, v.shape).astype(np.float32) for k, v in ws.mlp.get_params().items()})
+    out = []
+    for env in (None, "0"):
+        if env is None:
+            monkeypatch.delenv("G2G_ROWS", raising=False)
+        else:
+            monkeypatch.setenv("G2G_ROWS", env)
+        print(f"hard rows among learned starts {where} env={env}", flush=True)
+        B = _capi.Batch(_capi.Plan.from_grid(g.Ybus, g.pv, g.pq, g.slack), rows, precision=_capi.FP64)
+        B.set_sbus(S)
+        B.set_v(g.flat_start())
+        stats = B.solve_warm(ws.mlp, k_warm=4, growth=1.0, max_iter=10, tol=1e-8)
+        out.append((B.get_v(), *B.results(), stats))
+    (V, st, it, res, s1), (Vt, stt, itt, rest, s0) = out
+    np.testing.assert_array_equal(st, stt)
+    np.testing.assert_array_equal(it, itt)
+    assert s1["n_requeued"] == s0["n_requeued"] > 0
+    assert (st[where] != 0).all() and (np.delete(st, where) == 0).all()
+    np.testing.assert_array_equal(V[where], Vt[where])
+    np.testing.assert_array_equal(res[where], rest[where])
+    ok = st == 0
+    assert np.abs(V[ok] - Vt[ok]).max() < 1e-9
