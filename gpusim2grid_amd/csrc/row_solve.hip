@@ -254,7 +254,7 @@ __global__ __launch_bounds__(kRowMaxThreads) void k_row_solve(RowArgs<Real> a)
         bool decide = !a.skip_first;
         int iter = a.clock ? *a.clock + a.iter0 : a.iter0, st = kActive, n_upd = 0;
         double jm = 0.0;
-        int turn = 0, look = a.look;  // look: the update from which on a row must contract
+        int turn = 0, look = iter - it0 + a.look;  // look: the update from which on a row must contract
         if (tid == 0) {
             *slice_next = n_wave;
             red[0] = red[1] = 0ull;

@@ -16,11 +16,11 @@ constexpr int kRowRedBytes = 8 * 8;  // the workgroup's maxima (two sets of two)
 // callers keep getting the one they always got.  (Not in streamed rounds, where
 // a row's V moves on with every launch.)
 constexpr double kRowKeep = 1e-4;
-// Such a row is given up early: from its third update on, when an update does
-// not halve a residual above kRowKeep.  (By the oracle, from the flat start, 14
-// to 6,500 buses, injections scaled up to the last row that converges: every
-// row that converges halves it or better from the third update on, nearly all
-// others fail to by their fourth.)
+// Such a row is given up early: from its third update here (or since its
+// restart) on, when an update does not halve a residual above kRowKeep.  (By
+// the oracle, from the flat start, 14 to 6,500 buses, injections scaled up to
+// the last row that converges: every row that converges halves it or better
+// from the third update on, nearly all others fail to by their fourth.)
 constexpr int kRowLook = 3;
 constexpr double kRowContract = 0.5;
 constexpr int kRowGivenUp = 99;  // such a row's status inside the kernel
